@@ -45,6 +45,7 @@ struct KParams {
     const char *    kv;
     int64_t         kv_nb1, kv_nb3;
     int64_t         n_kv;
+    int             key_cap;       // keys a sequence can have at most (key_capacity below)
     const char *    mask;
     int64_t         mask_nb1, mask_ne0;
     int64_t         mask_nb3;      // bytes from one sequence's mask rows to the next one's (0: all sequences share the rows)
@@ -128,6 +129,13 @@ __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_ex
 
 __device__ __forceinline__ float xor32(float v) { return __shfl_xor(v, 32, 64); }
 
+
+// Keys a sequence can have at most: what the block table has room for, or the rows of a cache without one; under a mask no more than
+// its rows are wide (a key past their end counts as masked).
+inline int64_t key_capacity(const mla_attn_args * a) {
+    const int64_t n = a->block_table ? a->bt_stride * MLA_PAGE_TOKENS : a->n_kv;
+    return a->mask && a->mask_ne0 < n ? a->mask_ne0 : n;
+}
 
 // The pipelined decode kernel (mla_decode_kernel.hip); returns hipErrorInvalidValue for shapes it does not take.
 bool       decode_fast_applicable(const mla_attn_args * a);

@@ -171,12 +171,12 @@ template <typename KP> __device__ __forceinline__ void sched_first_piece(const K
     hdr[1] = base + (pos - first) * unit_tokens;
     hdr[2] = base + (piece_end - first) * unit_tokens;
     if (p.balanced == 1) {
-        const int len = min(p.seq_lens[it], (int) p.bt_stride * MLA_PAGE_TOKENS);
+        const int len = min(p.seq_lens[it], p.key_cap);
         hdr[2] = min(len, hdr[2]);
         hdr[3] = min(max(p.block_table[(int64_t) it * p.bt_stride + (pos - first)], 0), p.n_pool_pages - 1);
         hdr[7] = len;
     } else {
-        hdr[7] = (int) p.n_kv;
+        hdr[7] = p.key_cap;
     }
     hdr[4] = pos == first && piece_end == S[it + 1];
     hdr[5] = piece_end;
@@ -206,7 +206,7 @@ __device__ __forceinline__ void sched_prefix(const KParams & p) {
     __shared__ int S[2 * SCHED_MAX_SEQ + 8];
     const int t = threadIdx.x;
     int pages = 0;
-    if (t < p.n_units) pages = (max(min(p.seq_lens[t], (int) p.bt_stride * MLA_PAGE_TOKENS), 0) + MLA_PAGE_TOKENS - 1) / MLA_PAGE_TOKENS;
+    if (t < p.n_units) pages = (max(min(p.seq_lens[t], p.key_cap), 0) + MLA_PAGE_TOKENS - 1) / MLA_PAGE_TOKENS;
     sched_scan(S, pages, 0, p.n_units);
     if (t <= p.n_units) p.sched[t] = S[t];
     if (t == 0 && p.n_units == SCHED_MAX_SEQ) p.sched[SCHED_MAX_SEQ] = S[SCHED_MAX_SEQ];
@@ -340,7 +340,7 @@ __device__ __forceinline__ void decode_body() {
             const int * tab = (const int *) smem + (p.dual == 1 ? 2 * SCHED_MAX_SEQ : 0);
             tiles = tab[t]; base = tab[SCHED_MAX_SEQ + t];
         } else {
-            tiles = mask_item_tiles(p.mask_ext, t, p.n_units, (int) p.n_kv, base);
+            tiles = mask_item_tiles(p.mask_ext, t, p.n_units, p.key_cap, base);
         }
         sched_scan(sched, tiles, base, p.n_units);
         // Aligned schedule.  Equal runs of the tile list cross from one item into the next wherever they happen to, and a workgroup
@@ -387,7 +387,7 @@ __device__ __forceinline__ void decode_body() {
             first_piece[1] = __builtin_amdgcn_readfirstlane(b0 + (int) ((int64_t) k * u / w) * TILE_TOK);
             first_piece[2] = __builtin_amdgcn_readfirstlane(b0 + (int) ((int64_t) (k + 1) * u / w) * TILE_TOK);
             first_piece[4] = __builtin_amdgcn_readfirstlane(w == 1);
-            first_piece[7] = (int) p.n_kv;
+            first_piece[7] = p.key_cap;
             __syncthreads();   // (W is read; the tile buffers may be written)
         } else {
             int hdr[8];
@@ -404,7 +404,7 @@ __device__ __forceinline__ void decode_body() {
         int pages = 0, len = 0;
         if (t < p.n_units) {
             len   = p.seq_lens[t];
-            pages = (max(min(len, (int) p.bt_stride * MLA_PAGE_TOKENS), 0) + MLA_PAGE_TOKENS - 1) / MLA_PAGE_TOKENS;
+            pages = (max(min(len, p.key_cap), 0) + MLA_PAGE_TOKENS - 1) / MLA_PAGE_TOKENS;
         }
         sched_scan(sched, pages, len, p.n_units);
         if (bx == 0) {
@@ -454,11 +454,11 @@ __device__ __forceinline__ void decode_body() {
             const int first = sched[item], piece_end = min(sched[item + 1], run_end);
             if constexpr (MASK) {
                 const int base = sched[SCHED_MAX_SEQ + 8 + item];
-                seq_len  = (int) p.n_kv;
+                seq_len  = p.key_cap;
                 kv_begin = base + (run_pos - first) * TILE_TOK;
                 kv_end   = base + (piece_end - first) * TILE_TOK;
             } else {
-                seq_len  = min(sched[SCHED_MAX_SEQ + 8 + item], (int) p.bt_stride * MLA_PAGE_TOKENS);
+                seq_len  = min(sched[SCHED_MAX_SEQ + 8 + item], p.key_cap);
                 kv_begin = (run_pos - first) * MLA_PAGE_TOKENS;
                 kv_end   = min(seq_len, (piece_end - first) * MLA_PAGE_TOKENS);
             }
@@ -470,7 +470,7 @@ __device__ __forceinline__ void decode_body() {
         slot  = bx + item;
         split = 1;   // not the first split of anything: an empty piece writes nothing
     } else {
-        seq_len  = p.block_table ? min(p.seq_lens[b], (int) p.bt_stride * MLA_PAGE_TOKENS) : (int) p.n_kv;
+        seq_len  = p.block_table ? min(p.seq_lens[b], p.key_cap) : p.key_cap;
         kv_begin = split * p.split_tokens;
         kv_end   = min(seq_len, kv_begin + p.split_tokens);
         slot     = b * p.n_splits + split;
@@ -731,7 +731,7 @@ __global__ void __launch_bounds__(NTHREADS) mla_decode_dual_kernel(const KParams
     // (the tile buffers are not in use yet)  tab: tiles and first key of the key range of every token, then of every row block --
     // the body reads its items' from here; raw: the tokens' ranges as they are, for the merge; tot: the waves' sums
     int * tab = (int *) smem, * raw = tab + 4 * SCHED_MAX_SEQ, * tot = raw + 2 * SCHED_MAX_SEQ;
-    const int t = threadIdx.x, n_kv = (int) pb.n_kv;
+    const int t = threadIdx.x, n_kv = pb.key_cap;
     auto tiles_of = [&](int mlo, int mhi, int & base) {   // rounded outwards to tiles
         const int hi = min(n_kv, (mhi + TILE_TOK - 1) / TILE_TOK * TILE_TOK), lo = min(mlo / TILE_TOK * TILE_TOK, hi);
         base = lo;
@@ -778,7 +778,7 @@ __global__ void __launch_bounds__(NTHREADS) mla_decode_dual_kernel(const KParams
 constexpr int MASK_EXT_CHUNKS = 16;
 __device__ __forceinline__ void mask_extent_block_tokens(const KParams & p, int t0, int n_t, int chunk) {
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int n_kv = (int) p.n_kv;
+    const int n_kv = p.key_cap;
     const int n8 = n_kv / 8;
     const int g0 = (int) ((int64_t) n8 * chunk / MASK_EXT_CHUNKS), ng = (int) ((int64_t) n8 * (chunk + 1) / MASK_EXT_CHUNKS) - g0;
     constexpr int U = 4;
@@ -829,7 +829,7 @@ __device__ __forceinline__ void mask_extent_block(const KParams & p, int rb, int
         if (sub >= n_t) return;
         t0 += sub; n_t = 1; slot = t0;
     }
-    const int n_kv = (int) (p.block_table ? p.bt_stride * MLA_PAGE_TOKENS : p.n_kv);
+    const int n_kv = p.key_cap;
     const int n8 = n_kv / 8;   // groups of 8 mask values (16 bytes); n_kv is a multiple of 32 on this path
     const int g0 = (int) ((int64_t) n8 * chunk / MASK_EXT_CHUNKS), ng = (int) ((int64_t) n8 * (chunk + 1) / MASK_EXT_CHUNKS) - g0;
     // the (token, group) pairs of this sixteenth form one list, eight 16-byte loads per thread in flight: a loop over the tokens
@@ -907,7 +907,7 @@ __global__ void __launch_bounds__(NTHREADS) mla_mask_extent_wave_kernel(const KP
     if (rb >= n_rb) return;
     const int r0 = rb * 128, r1 = min(r0 + 127, p.n_rows - 1);
     const int t0 = r0 / p.n_head, n_t = r1 / p.n_head - t0 + 1;
-    const int n_kv = (int) (p.block_table ? p.bt_stride * MLA_PAGE_TOKENS : p.n_kv);
+    const int n_kv = p.key_cap;
     const int n8 = n_kv / 8;
     const int g0 = (int) ((int64_t) n8 * chunk / MASK_EXT_CHUNKS), ng = (int) ((int64_t) n8 * (chunk + 1) / MASK_EXT_CHUNKS) - g0;
     const int total = n_t * ng;   // (the launcher takes this form for at most 1024 (token, group) pairs per sixteenth)
@@ -1094,8 +1094,11 @@ bool decode_fast_applicable(const mla_attn_args * a) {
     if (a->kv_type != MLA_TYPE_Q8_0 && a->kv_nb1 != ROW_BYTES) return false;   // (the f16 copy of a Q8_0 cache is packed by construction)
     if (a->mask) {
         // whole tiles only (no key past n_kv is touched in a mask row), 32-bit offsets into the mask, 8-byte aligned loads
-        const int64_t n_kv = a->block_table ? a->bt_stride * MLA_PAGE_TOKENS : a->n_kv;
-        if (n_kv % TILE_TOK || a->mask_ne0 < n_kv || (a->mask_nb1 & 7) || ((uintptr_t) a->mask & 7)) return false;
+        // A mask row may be narrower than the cache -- a prompt chunk of several sequences brings rows as wide as the longest of them, its
+        // block table has room for whole pages: keys past the row's end count as masked, so the row's end is the cache's
+        // (2 sequences x 537 new tokens x 64 heads, rows of 544 over pages of 640: 1014 us on the general kernel, 172 us here).
+        const int64_t n_kv = key_capacity(a);
+        if (n_kv % TILE_TOK || (a->mask_nb1 & 7) || ((uintptr_t) a->mask & 7)) return false;
         if ((int64_t) a->n_tok * a->mask_nb1 >= (1ll << 31)) return false;
     }
     if (!(a->scale > 0.0f) || !(a->scale < INFINITY)) return false;
@@ -1217,7 +1220,7 @@ hipError_t launch_decode_fast(const KParams & kp_in, int kv_type, dim3 grid, hip
     // (a launch issued in two forms scans per query token: 16 layers for each of the tokens a row block can hold)
     // long mask rows -- a decode batch: the row spans the whole cache; a sixteenth of it is a block's worth of 16-byte groups from
     // 32768 keys on -- get a block per (token, sixteenth), shorter ones (a prompt chunk) a wave per token
-    const int ext_sub = kp.dual && kp.n_kv >= 32768 ? min(kp.n_tok, 127 / kp.n_head + 2) : 1;
+    const int ext_sub = kp.dual && kp.key_cap >= 32768 ? min(kp.n_tok, 127 / kp.n_head + 2) : 1;
     kp.mask_ext_in_pack = fold ? 1 : 0;
     kp.mask_ext_sub = ext_sub;
     const unsigned ext = fold ? MASK_EXT_CHUNKS * ext_sub : 0;
@@ -1233,7 +1236,7 @@ hipError_t launch_decode_fast(const KParams & kp_in, int kv_type, dim3 grid, hip
     else                              hipLaunchKernelGGL(mla_q_pack_kernel<0>, dim3(n_rb, n_seq + tok_layers, KSTEPS + extra + ext), dim3(NTHREADS), 0, st, kp);
     if (m && !fold && with_prepass && scan_mask) {
         // many row blocks with little to scan per (row block, sixteenth): 16 lanes per pair instead of a block
-        const int64_t n_kv_m = kp.block_table ? kp.bt_stride * MLA_PAGE_TOKENS : kp.n_kv;
+        const int64_t n_kv_m = kp.key_cap;
         const int64_t per_pair = (int64_t) (127 / kp.n_head + 2) * (n_kv_m / 8 / MASK_EXT_CHUNKS + 1);
         if (!kp.dual && n_rb * MASK_EXT_CHUNKS >= 1024 && per_pair <= 1024)
             hipLaunchKernelGGL(mla_mask_extent_wave_kernel, dim3(n_rb), dim3(NTHREADS), 0, st, kp, (int) n_rb);

@@ -990,7 +990,7 @@ int make_plan(const mla_attn_args * a, Plan * pl) {
     const int rc = validate(a);
     if (rc) return rc;
     const int64_t n_rows  = (int64_t) a->n_tok * a->n_head;
-    const int64_t max_len = a->block_table ? a->bt_stride * MLA_PAGE_TOKENS : a->n_kv;
+    int64_t max_len = a->block_table ? a->bt_stride * MLA_PAGE_TOKENS : a->n_kv;
     *pl = Plan{};
     // The replay of the reference's own arithmetic (mla_ref_scores_kernel, mla_ref_walk_kernel): asked for by flag, and taken by
     // itself for a Q8_0 cache of at most one page per sequence -- with so few keys one of them can carry a row, and then the
@@ -1006,7 +1006,7 @@ int make_plan(const mla_attn_args * a, Plan * pl) {
         pl->split_tokens = (int) max_len;
         return 0;
     }
-    if (decode_fast_applicable(a) && a->rows_per_wg == 0) { pl->variant = 2; pl->n_passes = a->dv == 576 ? 2 : 1; pl->ndb = 16; pl->wm = 4; pl->wd = 1; }
+    if (decode_fast_applicable(a) && a->rows_per_wg == 0) { max_len = key_capacity(a); pl->variant = 2; pl->n_passes = a->dv == 576 ? 2 : 1; pl->ndb = 16; pl->wm = 4; pl->wd = 1; }
     else if (a->dv == 576) { pl->n_passes = 2; pl->ndb = 9; pl->wm = 4; pl->wd = 1; }
     else {
         pl->n_passes = 1; pl->ndb = 16;
@@ -1058,8 +1058,8 @@ int make_plan(const mla_attn_args * a, Plan * pl) {
     if (pl->variant == 0 && a->mask) {
         // the general kernel visits only the key range the mask leaves open, when the extent pass can read the mask rows
         // (8-byte loads over whole groups of 8 keys)
-        const int64_t nk = a->block_table ? a->bt_stride * MLA_PAGE_TOKENS : a->n_kv;
-        if (nk % 8 == 0 && a->mask_ne0 >= nk && !(a->mask_nb1 & 7) && !((uintptr_t) a->mask & 7))
+        const int64_t nk = key_capacity(a);
+        if (nk % 8 == 0 && !(a->mask_nb1 & 7) && !((uintptr_t) a->mask & 7))
             pl->ws_maskext = (size_t) ((n_rows + 127) / 128) * 16 * 2 * sizeof(int);
     }
     // A paged decode batch (one row block per sequence, no mask) that needs KV splits anyway: the pipelined kernel's
@@ -1174,7 +1174,7 @@ static int launch_phases(const mla_attn_args * a, void * stream, int phases) {
 
     KParams kp{};
     kp.q = (const char *) a->q; kp.q_nb1 = a->q_nb1; kp.q_nb2 = a->q_nb2; kp.q_nb3 = a->q_nb3;
-    kp.kv = (const char *) a->kv; kp.kv_nb1 = a->kv_nb1; kp.kv_nb3 = a->kv_nb3; kp.n_kv = a->n_kv;
+    kp.kv = (const char *) a->kv; kp.kv_nb1 = a->kv_nb1; kp.kv_nb3 = a->kv_nb3; kp.n_kv = a->n_kv; kp.key_cap = (int) key_capacity(a);
     kp.mask = (const char *) a->mask; kp.mask_nb1 = a->mask_nb1; kp.mask_ne0 = a->mask_ne0; kp.mask_nb3 = 0;   // (shared by the sequences, ggml-cpu.c:12024)
     kp.block_table = a->block_table; kp.bt_stride = a->bt_stride; kp.seq_lens = a->seq_lens;
     kp.dst = a->dst; kp.dst_stride = a->dst_nb1 / 4;
