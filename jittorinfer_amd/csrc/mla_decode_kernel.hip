@@ -955,7 +955,8 @@ __device__ __forceinline__ bool pack_launch_extent_layer(const KParams & p) {
 // Q f32 -> the decode kernel's MFMA operand image, rounded to the KV type as ggml-cpu rounds it (ggml-cpu.c:12034-12035):
 // out[((seq*n_row_blocks + rb)*4 + wave)*36 + ks][lane] = 8 values of row rb*128 + wave*32 + lane%32,
 // columns 16*ks + 8*(lane/32) .. +7.  Rows past n_rows repeat the last row (their results are never stored);
-// a group of 32 rows that lies past n_rows entirely is left unwritten, its wave of the decode kernel neither loads nor computes.
+// in a sequence of one row block a group of 32 rows that lies past n_rows entirely is left unwritten: its wave of the decode kernel
+// has nothing to compute.
 // grid = (n_row_blocks, n_seq, 36 k-steps), block = 256: one 16-byte output per thread.
 // MODE 0: bf16 operands; 1: f16; 2: rounded to bf16 as for MODE 0, then written as f16 (exact inside the f16 range,
 // +-65504 beyond it) for the program that converts its bf16 tiles to f16.
@@ -994,7 +995,7 @@ __global__ void __launch_bounds__(NTHREADS) mla_q_pack_kernel(const KParams p) {
     const int ks = blockIdx.z;
     PackWhere w;
     if (!pack_where(p, wave, w)) return;
-    if (w.rb * 128 + w.wave * 32 >= w.n_rows) return;   // a wave of the decode kernel without a row: it computes nothing, its image is never used
+    if (w.n_rows <= 128 && w.wave * 32 >= w.n_rows) return;   // a wave of the decode kernel without a row that computes nothing: its image is never used
     const int row = min(w.rb * 128 + w.wave * 32 + rl, w.n_rows - 1);
     const int tq = row / p.n_head, head = row - tq * p.n_head;
     const float * qrow = (const float *) (p.q + (int64_t) tq * p.q_nb1 + (int64_t) head * p.q_nb2 + (int64_t) w.b * w.q_nb3) + 8 * g;
@@ -1150,11 +1151,15 @@ static hipError_t launch_variant(const KParams & kp, dim3 grid, hipStream_t st) 
 
 constexpr int64_t STREAM_CACHE_BYTES = 96ll << 20;   // (three times what the eight L2s hold)
 
+// Launches whose blocks of 128 rows are full, or of which at most the last one is not: its waves without rows compute on copies of the
+// last row (or on what the image holds) and nothing of theirs is stored.  The row-split program leaves such waves idle, but it is the slower one on every full
+// block, and it takes an operand image (2 sequences x 537 tokens x 64 heads, 64 rows over: 172 -> 117 us).  A single block of 65 to
+// 96 rows runs as fast on either (32 sequences x 8192 keys: 80 heads 101.6 / 100.7 us, 96 heads 102.3 / 103.4): it stays there.
 static bool decode_cs_applicable(const KParams & kp, int kv_type) {
     if (kv_type != MLA_TYPE_BF16 && kv_type != MLA_TYPE_F16) return false;
     if (kp.bf16_direct || kp.q_as_q8) return false;
     const int tail = kp.n_rows % 128;
-    return (tail == 0 || tail > 96) && kp.slot_rows < (1 << 22);
+    return (tail == 0 || tail > 96 || kp.n_rows > 128) && kp.slot_rows < (1 << 22);
 }
 
 // 33 .. 64 rows per sequence (a decode step of a model with 48 or 64 heads per device), no mask: the column-split program for two row
@@ -1192,8 +1197,8 @@ hipError_t launch_decode_fast(const KParams & kp_in, int kv_type, dim3 grid, hip
     const bool m = kp_in.mask != nullptr;
     // bf16 tiles are converted to f16 inside LDS unless the caller asks for the hi + lo program, or a single wave of a workgroup
     // has rows (16- and 32-head decode): one computing wave is not bound by its MFMAs, and the hi + lo program is the more exact
-    // column-split programs (every wave computes S for its own 32 rows and P.V for its own 128 columns): blocks of 128 rows in
-    // which all four waves have rows, not the Q8_0 expansion; bf16 K enters as bf16, so the Q image is the bf16 one
+    // column-split programs (every wave computes S for its own 32 rows and P.V for its own 128 columns): decode_cs_applicable, not the
+    // Q8_0 expansion; bf16 K enters as bf16, so the Q image is the bf16 one
     const bool cs = decode_cs_applicable(kp_in, kv_type), ks = decode_ks_applicable(kp_in, kv_type);
     const bool csh = !tok && decode_csh_applicable(kp_in, kv_type);
     const bool bf16_cvt = !cs && !csh && !kp_in.bf16_direct && kp_in.n_rows > 32;

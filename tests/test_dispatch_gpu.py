@@ -29,3 +29,17 @@ def test_mask_rows_narrower_than_the_block_table(gpu, k_type, n_head, n_new, n_o
     assert _plan_variant(gpu, q, pool, k_type, mask, bt, lens, scale=U.SCALE) == 2
     got = _run(gpu, q, pool, k_type, mask=mask, bt=bt, lens=lens, scale=U.SCALE)
     print(U.check(got[..., :512], _want(q, [s[:width] for s in seqs], k_type, mask), "narrow mask rows"))
+
+
+@pytest.mark.parametrize("k_type", [O.TYPE_BF16, O.TYPE_F16])
+@pytest.mark.parametrize("n_head,n_new", [(43, 3), (80, 2), (24, 8), (32, 7), (16, 17)])   # 129, 160, 192, 224, 272 rows
+@pytest.mark.parametrize("masked", [False, True])
+def test_row_blocks_of_which_the_last_is_not_full(gpu, k_type, n_head, n_new, masked):
+    """Two or three row blocks, 1 to 96 rows in the last: waves without rows beside blocks of 128."""
+    rng = np.random.default_rng(n_head * n_new)
+    n_kv = 224
+    q = rng.standard_normal((2, n_head, n_new, 576)).astype(np.float32)
+    k = U.encode_kv(rng.standard_normal((2, n_kv, 576)).astype(np.float32), k_type)
+    mask = _causal_mask(n_new, n_kv, n_kv) if masked else None
+    got = _run(gpu, q, k, k_type, mask=mask, scale=U.SCALE)
+    print(U.check(got[..., :512], _want(q, list(k), k_type, mask), "last row block not full"))
