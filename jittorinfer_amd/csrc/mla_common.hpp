@@ -73,7 +73,10 @@ struct KParams {
                                    // every query token as an item (the token form of a launch issued in two forms, see `dual`)
     int             n_wg;          //   workgroups (grid = (n_wg, 1, 1)); partial slot of workgroup v's piece of item i = v + i
     int             n_units;       //   items: sequences (1) / row blocks (2) / query tokens (3)
-    int             slot_rows;     // rows per partial slot: n_rows, or 128 with balanced == 2
+    int             slot_rows;     // rows per partial slot: n_rows, or 128 with balanced == 2 or tail_splits
+    int             tail_splits;   // masked launch of more row blocks than whole rounds of workgroups take: the (sequence, row block) items from
+    int             tail_first;    //   tail_first on (a multiple of 256) are split over tail_splits workgroups each, in partial slots of 128 rows; the
+                                   //   items before them have a workgroup each (grid = (tail_first + tail items * tail_splits, 1, 1)); 0: no tail
     int             n_seq_sched;   // sequences of the launch (grids of the pre-pack passes)
     int *           wg_first;      //   [n_wg][8] first piece of every workgroup (balanced == 1; workspace, written by the pre-pass).  Masked launches
                                    //   (balanced >= 2) keep there, written by the kernel's first workgroup for the combine pass: [1] = the schedule is

@@ -288,7 +288,8 @@ __device__ __forceinline__ void stage_q_rows(const KP & p, int b, int row0, int 
 typedef const __attribute__((address_space(4))) KParams KParamsArg;
 // STREAM (masked column-split and k-split programs): the build whose tile copies carry the non-temporal hint
 // RSBIAS (masked row-split programs of the f16 kinds: SRC_F16, SRC_BF16_CVT, SRC_Q8): the build with ALiBi slope and soft cap
-template <int KVT, bool MASK, int KOFF, bool OPAQUE, bool STREAM = false, bool RSBIAS = false>
+// TAIL: the launch has a tail of row blocks that several workgroups share (p.tail_splits)
+template <int KVT, bool MASK, int KOFF, bool OPAQUE, bool STREAM = false, bool RSBIAS = false, bool TAIL = false>
 __device__ __forceinline__ void decode_body() {
     static_assert(!RSBIAS || (MASK && (KVT == SRC_F16 || KVT == SRC_BF16_CVT || KVT == SRC_Q8)), "bias builds of the row-split programs");
     KParamsArg * p_ptr = (KParamsArg *) ((const __attribute__((address_space(4))) char *) __builtin_amdgcn_kernarg_segment_ptr() + KOFF);
@@ -303,7 +304,16 @@ __device__ __forceinline__ void decode_body() {
     // (sequence, row block) all read the same 147 KB Q operand image, so the dispatch index is remapped to put them on one
     // XCD: index i runs on XCD i % 8, and the i / 8-th workgroup of that XCD takes the tuple number (i % 8) * G / 8 + i / 8.
     int bx = blockIdx.x, by = blockIdx.y, bz = blockIdx.z;
-    {
+    bool tail = false;   // this workgroup has one of several pieces of a row block of the launch's tail
+    if constexpr (TAIL) {
+        const int n_rb = (p.n_rows + 127) / 128, id = blockIdx.x;
+        int item;
+        tail = id >= p.tail_first;
+        if (tail) { item = p.tail_first + (id - p.tail_first) / p.tail_splits; bx = (id - p.tail_first) % p.tail_splits; }
+        else      { item = (id & 7) * (p.tail_first >> 3) + (id >> 3); bx = 0; }   // neighbours share an XCD, as below
+        if (!tail && p.n_seq_sched == 1) item = (item & 1) ? p.tail_first - 1 - (item >> 1) : (item >> 1);   // in folded order, as below
+        bz = item / n_rb; by = item - bz * n_rb;
+    } else {
         const unsigned G = gridDim.x * gridDim.y * gridDim.z;
         if ((G & 7) == 0) {
             const unsigned id = (blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
@@ -313,7 +323,7 @@ __device__ __forceinline__ void decode_body() {
             // come -- would give the first XCD the shortest row blocks of a sequence and the last the longest (512 tokens x 128 heads
             // from an empty cache: 2 against 16 tiles).  The row blocks are therefore taken in folded order 0, R-1, 1, R-2, ...: any run
             // of an even number of them has the same number of keys as any other, and the blocks of one sequence still share an XCD.
-            if (MASK && gridDim.x == 1 && !p.balanced) by = (by & 1) ? (int) gridDim.y - 1 - (by >> 1) : (by >> 1);
+            if (MASK && !TAIL && gridDim.x == 1 && !p.balanced) by = (by & 1) ? (int) gridDim.y - 1 - (by >> 1) : (by >> 1);
         }
     }
 
@@ -436,8 +446,9 @@ __device__ __forceinline__ void decode_body() {
     asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane));
     const int tid = wave * 64 + lane, g = lane >> 5, rl = lane & 31;
     int b = bz, split = bx, slot = 0;
+    const int n_splits = tail ? p.tail_splits : p.n_splits;
     int seq_len, kv_begin, kv_end;
-    bool direct = p.n_splits == 1;   // this piece is the whole sequence / key range: final rows go to dst, there is nothing to combine
+    bool direct = n_splits == 1;   // this piece is the whole sequence / key range: final rows go to dst, there is nothing to combine
     int pg0_ready = -1;
     if (p.balanced) {
         int item;
@@ -473,13 +484,14 @@ __device__ __forceinline__ void decode_body() {
         seq_len  = p.block_table ? min(p.seq_lens[b], p.key_cap) : p.key_cap;
         kv_begin = split * p.split_tokens;
         kv_end   = min(seq_len, kv_begin + p.split_tokens);
-        slot     = b * p.n_splits + split;
+        slot     = tail ? (int) blockIdx.x - p.tail_first : b * p.n_splits + split;
     }
     const int row       = by * 128 + wave * 32 + rl;
     const bool row_valid = row < p.n_rows;
     const int64_t orow  = (int64_t) b * p.n_rows + row;
     // a partial slot holds p.slot_rows rows: all rows of the sequence (uniform splits), or the 128 of one row block
-    const int lrow      = p.balanced == 2 ? row - by * 128 : row;
+    const bool block_slots = p.balanced == 2 || tail;
+    const int lrow      = block_slots ? row - by * 128 : row;
     const int64_t prow  = (int64_t) slot * p.slot_rows + lrow;
 
     bool all_masked = false;  // this split holds keys, but none that a row of this block may attend to
@@ -490,7 +502,7 @@ __device__ __forceinline__ void decode_body() {
             mhi = max(mhi, p.mask_ext[(by * 16 + c) * 2 + 1]);
         }
         const int hi = min(seq_len, (mhi + TILE_TOK - 1) / TILE_TOK * TILE_TOK), lo = min(mlo / TILE_TOK * TILE_TOK, hi);
-        int chunk = ((hi - lo + p.n_splits - 1) / p.n_splits + TILE_TOK - 1) / TILE_TOK * TILE_TOK;
+        int chunk = ((hi - lo + n_splits - 1) / n_splits + TILE_TOK - 1) / TILE_TOK * TILE_TOK;
         kv_begin = lo + split * chunk;
         kv_end   = min(hi, kv_begin + chunk);
         if (split == 0 && kv_end <= kv_begin) kv_end = min(seq_len, kv_begin + TILE_TOK);  // no key at all: one masked tile, so that the rows come out NaN
@@ -500,11 +512,11 @@ __device__ __forceinline__ void decode_body() {
         // Nothing to read.  Only the first split of an empty sequence writes something: a NaN row, like the reference's
         // 0 * (1/0); other empty splits are skipped by the combine pass.  A split whose keys are all masked tells the
         // combine pass so (m = -inf).
-        if ((all_masked || (MASK && split > 0)) && p.n_splits > 1 && row_valid && g == 0) {
+        if ((all_masked || (MASK && split > 0)) && n_splits > 1 && row_valid && g == 0) {
             p.part_ml[prow * 2] = -INFINITY;
             p.part_ml[prow * 2 + 1] = 0.f;
         } else if (seq_len <= 0 && split == 0 && row_valid && g == 0) {
-            if (p.n_splits == 1) {
+            if (n_splits == 1) {
                 float * o = p.dst + orow * p.dst_stride;
                 for (int d = 0; d < 512; d++) o[p.v_col0 + d] = __builtin_nanf("");
             } else {
@@ -582,7 +594,7 @@ __device__ __forceinline__ void decode_body() {
 
     // column-split programs: every wave stores 128 columns of all 128 rows, so the output is described by scalars -- the block's
     // first row in dst (final rows) or in its partial slot, the byte pitch of f32 rows, and the number of rows that exist
-    const int lrow0 = p.balanced == 2 ? 0 : by * 128;
+    const int lrow0 = block_slots ? 0 : by * 128;
     const char * out_base = direct ? (const char *) (p.dst + ((int64_t) b * p.n_rows + by * 128) * p.dst_stride + p.v_col0)
                           : p.part_f32 ? (const char *) ((float *) p.part_o + ((int64_t) slot * p.slot_rows + lrow0) * p.dv_total)
                                        : (const char *) (p.part_o + pblock + (int64_t) lrow0 * 8);
@@ -716,8 +728,8 @@ __device__ __forceinline__ void decode_body() {
   }
 }
 
-template <int KVT, bool MASK, bool STREAM = false, bool RSBIAS = false>
-__global__ void __launch_bounds__(NTHREADS) mla_decode_kernel(const KParams) { decode_body<KVT, MASK, 0, false, STREAM, RSBIAS>(); }   // (the body reads the argument segment)
+template <int KVT, bool MASK, bool STREAM = false, bool RSBIAS = false, bool TAIL = false>
+__global__ void __launch_bounds__(NTHREADS) mla_decode_kernel(const KParams) { decode_body<KVT, MASK, 0, false, STREAM, RSBIAS, TAIL>(); }   // (the body reads the argument segment)
 
 // A masked launch of few heads issued in two forms (the launcher's comment tells why): pb describes it as row blocks of 128 rows
 // (balanced == 2), pt token by token (balanced == 3: every query token a sequence of one token, its mask row that sequence's
@@ -1140,12 +1152,12 @@ hipError_t launch_q8_to_f16(const char * src, int64_t src_nb1, int64_t src_nb3, 
     return hipGetLastError();
 }
 
-template <int KVT, bool MASK, bool STREAM = false, bool RSBIAS = false>
+template <int KVT, bool MASK, bool STREAM = false, bool RSBIAS = false, bool TAIL = false>
 static hipError_t launch_variant(const KParams & kp, dim3 grid, hipStream_t st) {
     static bool attr_done[MLA_MAX_DEVICES];
-    const hipError_t e = raise_lds_limit((const void *) mla_decode_kernel<KVT, MASK, STREAM, RSBIAS>, attr_done);
+    const hipError_t e = raise_lds_limit((const void *) mla_decode_kernel<KVT, MASK, STREAM, RSBIAS, TAIL>, attr_done);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((mla_decode_kernel<KVT, MASK, STREAM, RSBIAS>), grid, dim3(NTHREADS), (size_t) lds_total(KVT), st, kp);
+    hipLaunchKernelGGL((mla_decode_kernel<KVT, MASK, STREAM, RSBIAS, TAIL>), grid, dim3(NTHREADS), (size_t) lds_total(KVT), st, kp);
     return hipGetLastError();
 }
 
@@ -1281,6 +1293,12 @@ hipError_t launch_decode_fast(const KParams & kp_in, int kv_type, dim3 grid, hip
         if (ks) return kv_type == MLA_TYPE_F16 ? launch_variant<SRC_F16_KSB, true>(kp, grid, st) : launch_variant<SRC_BF16_KSB, true>(kp, grid, st);
         if (cs) return kv_type == MLA_TYPE_F16 ? launch_variant<SRC_F16_CSB, true>(kp, grid, st) : launch_variant<SRC_BF16_CSB, true>(kp, grid, st);
         return kv_type == MLA_TYPE_F16 ? launch_variant<SRC_F16, true, false, true>(kp, grid, st) : launch_variant<SRC_BF16_CVT, true, false, true>(kp, grid, st);
+    }
+    if (kp.tail_splits) {   // (make_plan gives the others no tail)
+        if (!m || bias || kp.q_as_q8 || kp.balanced || kp.n_splits != 1) return hipErrorInvalidValue;
+        if (kv_type == MLA_TYPE_Q8_0) return launch_variant<SRC_Q8, true, false, false, true>(kp, grid, st);
+        if (!cs || !q_in_kernel) return hipErrorInvalidValue;
+        return kv_type == MLA_TYPE_F16 ? launch_variant<SRC_F16_CSQ, true, false, false, true>(kp, grid, st) : launch_variant<SRC_BF16_CSQ, true, false, false, true>(kp, grid, st);
     }
     if (kv_type == MLA_TYPE_Q8_0) return m ? launch_variant<SRC_Q8, true>(kp, grid, st) : launch_variant<SRC_Q8, false>(kp, grid, st);
     if (ks && m && stream) return kv_type == MLA_TYPE_F16 ? launch_variant<SRC_F16_KS, true, true>(kp, grid, st) : launch_variant<SRC_BF16_KS, true, true>(kp, grid, st);

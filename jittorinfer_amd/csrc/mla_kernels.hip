@@ -421,9 +421,17 @@ __global__ void __launch_bounds__(NTHREADS) mla_attn_tile_kernel(const KParams p
 // nvalid < 0: one workgroup had the whole item and wrote the final rows itself.
 // A launch issued in two forms (p.dual; the combine pass gets the row-block form's parameters): p.form tells which one ran; in the
 // token form an item is a query token and a slot holds its n_head rows.
+// TAIL: a launch with a tail (p.tail_splits; partials of the tail's row blocks only).
+template <bool TAIL = false>
 __device__ __forceinline__ void partial_slots(const KParams & p, int b, int row, int seq_len, int & slot0, int & nvalid, int & lrow, int & slot_rows) {
     lrow = row;
     slot_rows = p.slot_rows;
+    if constexpr (TAIL) {
+        slot0  = (b * ((p.n_rows + 127) / 128) + row / 128 - p.tail_first) * p.tail_splits;
+        nvalid = p.tail_splits;
+        lrow   = row % 128;
+        return;
+    }
     if (!p.balanced) {
         nvalid = (seq_len + p.split_tokens - 1) / p.split_tokens;
         nvalid = p.rel_splits ? p.n_splits : min(nvalid, p.n_splits);
@@ -449,21 +457,33 @@ __device__ __forceinline__ void partial_slots(const KParams & p, int b, int row,
     if (nvalid == 1) nvalid = -1;
 }
 
+// The row a thread of a combine pass merges.  A launch with a tail has partials of its tail's row blocks only: the pass runs over those
+// (b = 0, rows counted from the first of them).  False: there is no such row.
+template <bool TAIL>
+__device__ __forceinline__ bool combine_row(const KParams & p, int & b, int & row) {
+    if constexpr (TAIL) {
+        const int n_rb = (p.n_rows + 127) / 128, item = p.tail_first + row / 128;
+        b   = item / n_rb;
+        row = (item - b * n_rb) * 128 + row % 128;
+    }
+    return row < p.n_rows;
+}
+
 // Log-sum-exp merge of the split-K partials: out = sum_c (O_c/l_c) l_c 2^(m_c - M) / sum_c l_c 2^(m_c - M).
 // Partials hold O_c/l_c as f16, laid out [seq][split][column/8][row][8].  One thread = one row and two groups of 8 columns 128
 // columns apart: 16-byte loads, splits in groups of 8 so that all the loads of a group (8 (m, l) pairs, 16 partial chunks) are in
 // flight together, and the weights of a group of splits are worked out once for both column groups.  A wave covers 16 rows x 4
 // column groups (twice): it reads runs of 256 bytes (16 rows of one column group are contiguous in the partial layout) and writes
 // 128 contiguous bytes per row.  grid = (ceil(rows/16), ceil(dv/256), n_seq), block = 256 = 16 rows x 16 column groups (x 2).
+template <bool TAIL>
 __global__ void __launch_bounds__(256) mla_attn_combine_kernel(const KParams p) {
-    const int b = blockIdx.z;
-    const int row = blockIdx.x * 16 + (threadIdx.x & 15);
+    int b = blockIdx.z, row = blockIdx.x * 16 + (threadIdx.x & 15);
     const int cg  = blockIdx.y * 32 + (threadIdx.x >> 4);
+    if (!combine_row<TAIL>(p, b, row) || cg * 8 >= p.dv_total) return;
     const int seq_len = p.block_table ? min(p.seq_lens[b], (int) p.bt_stride * MLA_PAGE_TOKENS) : (int) p.n_kv;
-    if (row >= p.n_rows || cg * 8 >= p.dv_total) return;
     const bool two = (cg + 16) * 8 < p.dv_total;   // the second column group exists
     int slot0, nvalid, lrow, slot_rows;
-    partial_slots(p, b, row, seq_len, slot0, nvalid, lrow, slot_rows);
+    partial_slots<TAIL>(p, b, row, seq_len, slot0, nvalid, lrow, slot_rows);
     if (nvalid < 0) return;
 
     const float2 *   ml = (const float2 *) p.part_ml + (int64_t) slot0 * slot_rows + lrow;
@@ -640,15 +660,16 @@ __device__ __forceinline__ void combine_f32_row(const float2 * ml, const float *
     *(f32x4 *) dst = f32x4{ o.x * inv, o.y * inv, o.z * inv, o.w * inv };
 }
 
+template <bool TAIL>
 __global__ void __launch_bounds__(256) mla_attn_combine_f32_kernel(const KParams p, int groups_per_row) {
-    const int b = blockIdx.z;
     const int rows_per_block = 256 / groups_per_row;
-    const int row = blockIdx.x * rows_per_block + threadIdx.x / groups_per_row;
+    int b = blockIdx.z, row = blockIdx.x * rows_per_block + threadIdx.x / groups_per_row;
     const int cg  = threadIdx.x % groups_per_row;
+    if (!combine_row<TAIL>(p, b, row)) return;
     const int seq_len = p.block_table ? min(p.seq_lens[b], (int) p.bt_stride * MLA_PAGE_TOKENS) : (int) p.n_kv;
-    if (row >= p.n_rows || (int) threadIdx.x >= rows_per_block * groups_per_row || cg * 4 >= p.dv_total) return;
+    if ((int) threadIdx.x >= rows_per_block * groups_per_row || cg * 4 >= p.dv_total) return;
     int slot0, nvalid, lrow, slot_rows;
-    partial_slots(p, b, row, seq_len, slot0, nvalid, lrow, slot_rows);
+    partial_slots<TAIL>(p, b, row, seq_len, slot0, nvalid, lrow, slot_rows);
     if (nvalid < 0) return;
     const float2 * ml = (const float2 *) p.part_ml + (int64_t) slot0 * slot_rows + lrow;
     const float *  po = (const float *) p.part_o + ((int64_t) slot0 * slot_rows + lrow) * p.dv_total + cg * 4;
@@ -929,6 +950,7 @@ struct Plan {
     int    part_f32;
     int    balanced, n_wg, n_units;   // balanced schedule of the pipelined kernel (1: ragged paged decode, 2: masked launch)
     int    dual;                      // the masked launch is issued in two forms, see token_form_candidate
+    int    tail_first, tail_splits;   // masked launch beyond whole rounds of workgroups: see masked_splits
     int    seq_sorted;                // paged decode of more than 256 sequences: workgroups take the sequences longest first
 };
 
@@ -986,6 +1008,30 @@ static size_t token_image_bytes(const mla_attn_args * a) {
     return a->kv_type == MLA_TYPE_Q8_0 || a->n_head > 32 ? decode_fast_qpack_bytes(a->n_tok, 1) : 0;
 }
 
+// How long a masked launch (a prompt chunk) takes when `splits` workgroups share the keys of every row block: n_items = sequences x row
+// blocks of n_tiles 32-key tiles at most, in microseconds.  Fitted to launches measured on one box: a tile takes 1.33 us with few CUs
+// busy and 1.83 with all 256 (the chip's power limit), a workgroup 20 us beside its tiles (operands in, rows out, the scan of the
+// mask ahead), the pass that packs the operands of split row blocks and the merge of their partial rows 5 us + 0.1 per row block +
+// 0.01 per piece.  Measured: 8 row blocks x 94 tiles in 12 / 24 pieces each 40.7 / 35.2 us, 32 x 17 in 1 / 5 45.8 / 32.5, 108 x 32 in 2 / 3
+// 67.2 / 85.1 (3: a second round of workgroups), 108 x 103 in 2 / 3 126 / 162, 128 x 72 in 2 106, 26 x 129 in 9 59.4, 26 x 7 in 1 / 2 31.4 / 38.5.
+static double masked_split_cost(int64_t n_items, int64_t n_tiles, int64_t splits) {
+    const int64_t pieces = n_items * splits, rounds = (pieces + 255) / 256;
+    const double  busy = std::min(1.0, (double) pieces / 256), tile = 1.33 + 0.5 * busy;
+    return rounds * ((double) ((n_tiles + splits - 1) / splits) * tile + 20.0) + (splits > 1 ? 5.0 + 0.1 * n_items + 0.01 * pieces : 0.0);
+}
+static int64_t masked_splits(int64_t n_items, int64_t n_tiles, int64_t most) {
+    int64_t best = 1;
+    for (int64_t s = 2; s <= most && s <= n_tiles; s++)
+        if (masked_split_cost(n_items, n_tiles, s) < masked_split_cost(n_items, n_tiles, best)) best = s;
+    return best;
+}
+// One sequence in a contiguous cache, whose split form is the schedule that deals out equal runs of tiles: worth it from this many on.
+// 16 heads, a workgroup per row block / runs dealt out: 8 row blocks x 18 tiles 45.0 / 42.8 us, 32 x 8 33.3 / 43.8, 64 x 16 43.1 / 47.2, 64 x 32
+// 64.8 / 49.9, 128 x 64 110 / 99, 160 x 40 79 / 163, 160 x 168 252 / 236, 192 x 112 187 / 193, 250 x 63 119 / 281, 250 x 319 581 / 624.
+static bool masked_worth_dealing(int64_t n_items, int64_t n_tiles) {
+    return n_items <= 8 ? n_tiles > 4 : n_tiles * (1280 - 6 * n_items) > 15360;   // (2 x 10 35.1 / 25.2, 4 x 5 28.1 / 24.9, 8 x 6 29.6 / 28.2, 16 x 8 33.3 / 33.9)
+}
+
 int make_plan(const mla_attn_args * a, Plan * pl) {
     const int rc = validate(a);
     if (rc) return rc;
@@ -1026,6 +1072,20 @@ int make_plan(const mla_attn_args * a, Plan * pl) {
         const int64_t wgs = (int64_t) a->n_seq * pl->n_row_blocks;
         splits = (256 + wgs - 1) / wgs;
         if (pl->wd > 1) splits *= 2;  // small-row shapes leave room for two workgroups per CU
+        if (pl->variant == 2 && a->mask) {
+            const int64_t n_tiles = (max_len + TILE_TOK - 1) / TILE_TOK;
+            if (n_rows <= 32)   splits = std::max<int64_t>(256 / wgs, 1);   // (the k-split program: short pieces, and no second round for the rest)
+            else if (a->n_seq == 1 && !a->block_table) { if (!masked_worth_dealing(wgs, n_tiles)) splits = 1; }
+            else if (wgs < 256) splits = masked_splits(wgs, n_tiles, 32);
+            // More row blocks than whole rounds of 256 take: the ones left over would have the chip to themselves with most of it idle
+            // (333 row blocks x 130 tiles: the 77 of the second round took nearly as long as the 256 of the first).  They are split, the
+            // others not: 449 -> 376 us; 300 x 50 tiles 172 -> 143 us, 280 x 259 848 -> 575 us, 400 x 138 464 -> 454 us.
+            if (wgs > 256 && wgs % 256 && !(a->flags & (MLA_FLAG_UNIFORM_SPLITS | MLA_FLAG_BF16_DIRECT)) && decode_fast_q8_copy_rows(a) == 0 &&
+                a->logit_softcap == 0.0f && !(a->max_bias > 0.0f)) {   // (what the tail builds of the kernel take)
+                const int64_t n_tail = wgs % 256, best = masked_splits(n_tail, n_tiles, 8);
+                if (best > 1) { pl->tail_first = (int) (wgs - n_tail); pl->tail_splits = (int) best; }
+            }
+        }
     }
     // with a block table that kernel indexes at most 64 pages per split (63 with a mask, whose splits need not start on a page boundary)
     const int64_t max_pages = pl->variant == 2 && a->mask ? 63 : 64;
@@ -1051,6 +1111,7 @@ int make_plan(const mla_attn_args * a, Plan * pl) {
             pl->n_splits     = (int) ((n_tiles + tiles_per_split - 1) / tiles_per_split);
         }
     }
+    if (pl->n_splits > 1) pl->tail_first = pl->tail_splits = 0;   // (a paged launch whose sequences need splits anyway)
     pl->lds_bytes    = pl->variant == 2 ? decode_fast_lds_bytes(decode_fast_q8_copy_rows(a) > 0 ? MLA_TYPE_F16 : a->kv_type) : 2 * TILE_BYTES + (a->kv_type == MLA_TYPE_Q8_0 ? Q8_TILE_RAW : 0);
     if (pl->variant == 2) pl->ws_qpack = decode_fast_qpack_bytes(a->n_seq, pl->n_row_blocks);
     if (pl->variant == 2) { pl->kvcopy_rows = decode_fast_q8_copy_rows(a); pl->ws_kvcopy = (size_t) pl->kvcopy_rows * ROW_BYTES; }
@@ -1094,13 +1155,14 @@ int make_plan(const mla_attn_args * a, Plan * pl) {
         pl->ws_qpack  += token_image_bytes(a);
         pl->ws_sched   = (size_t) ((std::max(pl->n_units, a->n_tok) + 1 + 63) / 64 * 64 + pl->n_wg * 8) * sizeof(int);
     }
-    if (pl->n_splits > 1) {
+    if (pl->n_splits > 1 || pl->tail_splits) {
         // f32 partials while they are small (no second rounding of O on top of the MFMA operands' one), f16 beyond: there the
         // partial traffic counts, and the rounding (2^-12 relative per split) is averaged over long contexts
         // (the two forms of a launch issued in both share the area: the token form's n_wg + n_tok slots of n_head <= 32 rows fit
         // into the row-block form's n_wg + n_units slots of 128 rows)
-        const size_t n_slots = pl->balanced ? (size_t) pl->n_wg + pl->n_units : (size_t) a->n_seq * pl->n_splits;
-        const size_t slot_rows = pl->balanced == 2 ? 128 : (size_t) n_rows;
+        const size_t n_tail  = (size_t) a->n_seq * pl->n_row_blocks - pl->tail_first;
+        const size_t n_slots = pl->tail_splits ? n_tail * pl->tail_splits : pl->balanced ? (size_t) pl->n_wg + pl->n_units : (size_t) a->n_seq * pl->n_splits;
+        const size_t slot_rows = pl->balanced == 2 || pl->tail_splits ? 128 : (size_t) n_rows;
         const size_t n_part = n_slots * slot_rows * (pl->variant == 2 ? 512 : a->dv);
         pl->part_f32   = n_part * sizeof(float) <= ((size_t) 32 << 20);
         pl->ws_part_o  = n_part * (pl->part_f32 ? sizeof(float) : sizeof(_Float16));
@@ -1159,6 +1221,7 @@ int mla_attn_plan(const mla_attn_args * args, mla_attn_plan_info * out) {
     out->lds_bytes    = (int64_t) pl.lds_bytes;
     out->balanced     = pl.dual ? 4 : pl.balanced;
     out->n_workgroups = pl.balanced ? pl.n_wg : pl.n_splits * pl.n_row_blocks * a_n_seq;
+    if (pl.tail_splits) out->n_workgroups = pl.tail_first + (pl.n_row_blocks * a_n_seq - pl.tail_first) * pl.tail_splits;
     return 0;
 }
 
@@ -1195,7 +1258,8 @@ static int launch_phases(const mla_attn_args * a, void * stream, int phases) {
     kp.rel_splits = a->mask != nullptr && (pl.variant == 2 || pl.ws_maskext > 0);
     kp.balanced = pl.balanced; kp.n_wg = pl.n_wg; kp.n_seq_sched = a->n_seq; kp.n_units = pl.n_units;
     kp.bf16_direct = (a->flags & MLA_FLAG_BF16_DIRECT) ? 1 : 0;
-    kp.slot_rows = pl.balanced == 2 ? 128 : kp.n_rows;
+    kp.slot_rows = pl.balanced == 2 || pl.tail_splits ? 128 : kp.n_rows;
+    kp.tail_first = pl.tail_first; kp.tail_splits = pl.tail_splits;
     kp.part_ml = (float *) (ws + align256(pl.ws_part_o));
     float * scores = (float *) (ws + align256(pl.ws_part_o) + align256(pl.ws_part_ml));
     kp.q_pack = ws + align256(pl.ws_part_o) + align256(pl.ws_part_ml) + align256(pl.ws_scores);
@@ -1233,6 +1297,8 @@ static int launch_phases(const mla_attn_args * a, void * stream, int phases) {
 
     dim3 grid((unsigned) pl.n_splits, (unsigned) pl.n_row_blocks, (unsigned) a->n_seq);
     if (pl.balanced) grid = dim3((unsigned) pl.n_wg, 1, 1);
+    const int n_tail = a->n_seq * pl.n_row_blocks - pl.tail_first;   // row blocks of the tail, when there is one
+    if (pl.tail_splits) grid = dim3((unsigned) (pl.tail_first + n_tail * pl.tail_splits), 1, 1);
     int kv_type = a->kv_type;
     if (pl.kvcopy_rows > 0) {
         // Q8_0 cache + mask that the Q8_0 wave program cannot copy as raw tiles: expand the cache to f16 rows (a pre-pass like
@@ -1252,7 +1318,8 @@ static int launch_phases(const mla_attn_args * a, void * stream, int phases) {
         if (e != hipSuccess) return (int) e;
     }
     auto combine = [&](int dv) -> int {
-        const int splits_per_row = pl.balanced ? (pl.n_wg + pl.n_units - 1) / pl.n_units : pl.n_splits;
+        const unsigned c_rows = pl.tail_splits ? (unsigned) n_tail * 128 : (unsigned) kp.n_rows, c_seq = pl.tail_splits ? 1 : (unsigned) a->n_seq;
+        const int splits_per_row = pl.tail_splits ? pl.tail_splits : pl.balanced ? (pl.n_wg + pl.n_units - 1) / pl.n_units : pl.n_splits;
         if (pl.part_f32 && splits_per_row > 32) {   // (one or two sequences: the waves of a block share the walk over a row's splits)
             dim3 gw((unsigned) kp.n_rows, (unsigned) ((dv / 4 + 63) / 64), (unsigned) a->n_seq);
             hipLaunchKernelGGL(mla_attn_combine_f32_wide_kernel, gw, dim3(256), 0, st, kp);
@@ -1260,8 +1327,9 @@ static int launch_phases(const mla_attn_args * a, void * stream, int phases) {
         }
         if (pl.part_f32) {
             const int groups = dv / 4, rows_per_block = 256 / groups;   // 128 -> 2 rows, 144 -> 1 row
-            dim3 g((unsigned) ((kp.n_rows + rows_per_block - 1) / rows_per_block), 1, (unsigned) a->n_seq);
-            hipLaunchKernelGGL(mla_attn_combine_f32_kernel, g, dim3(256), 0, st, kp, groups);
+            dim3 g((c_rows + rows_per_block - 1) / rows_per_block, 1, c_seq);
+            auto kern = pl.tail_splits ? mla_attn_combine_f32_kernel<true> : mla_attn_combine_f32_kernel<false>;
+            hipLaunchKernelGGL(kern, g, dim3(256), 0, st, kp, groups);
             return (int) hipGetLastError();
         }
         // rows with many splits (few long sequences): four lanes share the walk over a row's splits
@@ -1275,8 +1343,9 @@ static int launch_phases(const mla_attn_args * a, void * stream, int phases) {
             hipLaunchKernelGGL(mla_attn_combine_wide_kernel<4>, gw, dim3(256), 0, st, kp);
             return (int) hipGetLastError();
         }
-        dim3 g((unsigned) ((kp.n_rows + 15) / 16), (unsigned) ((dv + 255) / 256), (unsigned) a->n_seq);
-        hipLaunchKernelGGL(mla_attn_combine_kernel, g, dim3(256), 0, st, kp);
+        dim3 g((c_rows + 15) / 16, (unsigned) ((dv + 255) / 256), c_seq);
+        auto kern = pl.tail_splits ? mla_attn_combine_kernel<true> : mla_attn_combine_kernel<false>;
+        hipLaunchKernelGGL(kern, g, dim3(256), 0, st, kp);
         return (int) hipGetLastError();
     };
     if (pl.variant == 2) {
@@ -1293,7 +1362,7 @@ static int launch_phases(const mla_attn_args * a, void * stream, int phases) {
             }
             // the partials of a pass are consumed before the next pass overwrites them; a combine-only call finishes the last pass
             const bool last = pass + 1 == pl.n_passes;
-            if (pl.n_splits > 1 && ((phases & 1) ? (!last || (phases & 2)) : (last && (phases & 2)))) {
+            if ((pl.n_splits > 1 || pl.tail_splits) && ((phases & 1) ? (!last || (phases & 2)) : (last && (phases & 2)))) {
                 const int rc2 = combine(512);
                 if (rc2) return rc2;
             }

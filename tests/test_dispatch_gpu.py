@@ -43,3 +43,44 @@ def test_row_blocks_of_which_the_last_is_not_full(gpu, k_type, n_head, n_new, ma
     mask = _causal_mask(n_new, n_kv, n_kv) if masked else None
     got = _run(gpu, q, k, k_type, mask=mask, scale=U.SCALE)
     print(U.check(got[..., :512], _want(q, list(k), k_type, mask), "last row block not full"))
+
+
+@pytest.mark.parametrize("k_type", [O.TYPE_BF16, O.TYPE_F16, O.TYPE_Q8_0])
+@pytest.mark.parametrize("n_seq,n_head,n_new,n_old,dv", [(1, 128, 257, 350, 512), (1, 128, 290, 352, 576), (1, 48, 693, 300, 512), (3, 16, 691, 250, 512)])
+def test_row_blocks_left_over_from_whole_rounds_are_split(gpu, k_type, n_seq, n_head, n_new, n_old, dv):
+    """257, 290, 260 and 3 x 87 row blocks: the 1, 34, 4 and 5 beyond 256 are split over several workgroups each (paged, several sequences
+    of different lengths: the tail lies in the last one).  One token of the tail sees no key: NaN rows.  Checked on sampled rows, the
+    tail's among them, and everywhere against the launch that does not split (same arithmetic but for the merge: f16 or f32 partials,
+    within the tolerance of the oracle)."""
+    import torch
+    import jittorinfer_amd as J
+    rng = np.random.default_rng(n_new + n_seq)
+    lens = [n_old + n_new - 40 * b for b in range(n_seq)]
+    q8s = 1.0 / 32 if k_type == O.TYPE_Q8_0 else None
+    width = (max(lens) + 31) // 32 * 32
+    q = rng.standard_normal((n_seq, n_head, n_new, 576)).astype(np.float32)
+    if n_seq > 1:
+        pool, bt, seqs = U.make_paged(rng, lens, k_type, q8_scale=q8s)
+        kw = dict(bt=bt, lens=lens)
+    else:
+        pool = U.encode_kv(rng.standard_normal((1, width, 576)).astype(np.float32), k_type, q8_scale=q8s)
+        seqs, kw = [pool[0]], {}
+    mask = _causal_mask(n_new, max(lens), width).copy()
+    mask[n_new - 1] = 0xfc00
+    tq = torch.from_numpy(q).to(gpu)
+    pkw = dict(mask=torch.from_numpy(mask.view(np.float16)).to(gpu), scale=U.SCALE)
+    if n_seq > 1:
+        pkw.update(block_table=torch.from_numpy(bt).to(gpu), seq_lens=torch.tensor(lens, dtype=torch.int32, device=gpu))
+    tp = torch.from_numpy(pool.view(np.int16) if pool.dtype == np.uint16 else pool).to(gpu)
+    n_items = n_seq * ((n_head * n_new + 127) // 128)
+    info = J.plan(tq, tp, k_type, dv=dv, **pkw)
+    assert info["variant"] == 2 and info["n_splits"] == 1 and info["n_workgroups"] > n_items > 256, info
+    assert J.plan(tq, tp, k_type, dv=dv, flags=J.MLA_FLAG_UNIFORM_SPLITS, **pkw)["n_workgroups"] == n_items
+    got = _run(gpu, q, pool, k_type, dv=dv, mask=mask, scale=U.SCALE, **kw)[..., :dv]
+    one = _run(gpu, q, pool, k_type, dv=dv, mask=mask, scale=U.SCALE, flags=J.MLA_FLAG_UNIFORM_SPLITS, **kw)[..., :dv]
+    print(U.check(got, one, "split against unsplit"))
+    for b in range(n_seq):
+        for t in (0, n_new // 2, n_new - 3, n_new - 2, n_new - 1):
+            want = (O.flash_attn_ext_f64 if k_type == O.TYPE_F16 else O.flash_attn_ext)(
+                q[b:b + 1, :, t:t + 1], seqs[b][None, :width], k_type, dv=dv, mask=np.ascontiguousarray(mask[t:t + 1, :len(seqs[b])]), scale=U.SCALE)
+            print(b, t, U.check(got[b:b + 1, t:t + 1], want, "sequence %d token %d" % (b, t)))
