@@ -1306,12 +1306,16 @@ def main():
     e("s_nop 1")
     e("s_and_b64 exec, exec, vcc")
     # O^T block i, element 4j+c is column 32 i + 8 j + 4 g + c.
-    # Final output (FLG bit 0): row-major rows of dst; the out pointer already includes the 4*g float offset.
+    # FLG bit 0: f32.  Final output: row-major rows of dst, the out pointer already includes the 4*g float offset.  Partials (FLG bit 7
+    # too): layout [column/4][row][4], the out pointer already includes row*16 bytes and g column groups; a step (i, j) is two of them.
     # Split-K partial: f16, layout [column/8][row][8] so that the 64 lanes of a wave write 512 contiguous bytes;
     # the out pointer already includes row*16 + g*8 bytes and every (i, j) step advances it by n_rows*16 bytes.
     lab_pstore, lab_sdone = label("pstore"), label("sdone")
     e("s_bitcmp1_b32 %s, 0" % s(FLG))
     e("s_cbranch_scc0 %s" % lab_pstore)
+    e("s_lshl_b32 %s, %s, 1" % (s(S0), s(OSTR)))
+    e("s_bitcmp1_b32 %s, 7" % s(FLG))
+    e("s_cselect_b32 %s, %s, 32" % (s(S0), s(S0)))
     for i in range(16):
         for j in range(4):
             r = T[4] if (i * 4 + j) % 2 == 0 else SA  # alternate two 4-register staging groups
@@ -1319,7 +1323,10 @@ def main():
                 e("v_accvgpr_read_b32 %s, %s" % (v(r + c), a(16 * i + 4 * j + c)))
             for c in range(4):
                 e("v_mul_f32 %s, %s, %s" % (v(r + c), v(r + c), v(T[2])))
-            e("global_store_dwordx4 %s, %s, off offset:%d" % (v(OPTR, 2), v(r, 4), (32 * i + 8 * j) * 4))
+            e("global_store_dwordx4 %s, %s, off" % (v(OPTR, 2), v(r, 4)))
+            e("v_add_co_u32 %s, vcc, %s, %s" % (v(OPTR), s(S0), v(OPTR)))
+            e("s_nop 1")
+            e("v_addc_co_u32 %s, vcc, 0, %s, vcc" % (v(OPTR + 1), v(OPTR + 1)))
     e("s_branch %s" % lab_sdone)
     e("%s:" % lab_pstore)
     # partial: O / l of this split as f16, layout [column/8][row][8 halves]; T[2] holds 1/l here as well

@@ -101,6 +101,7 @@ RSC, ONES, OSTR, QP, OB, MLB, RSTR, NRV = 72, 74, 75, 76, 78, 80, 82, 83
 W4, WOFS, FADR, PGZ, SPITCH, SCLS = 84, 85, 86, 87, 88, 89
 VM = [90, 92, 94, 96]   # epilogue: lanes whose row of row block hb exists
 SB = 98                 # epilogue: running store base
+CSTR = 88               # epilogue: bytes from one group of 4 columns to the next (SPITCH's register)
 # LDS-DMA loads (the epilogue's row masks take these registers afterwards): wave * bytes a wave copies per tile; the four clamp
 # offsets of the current tile; the first of them for the last tile of the piece; number of tiles - 1
 WDMA, CL, LAST0, NTM1 = 90, [91, 92, 93, 94], 95, 96
@@ -1138,17 +1139,23 @@ def epilogue(nhb):
     lab_pstore, lab_sdone = label("pstore"), label("sdone")
     e("s_bitcmp1_b32 %s, 0" % s(FLG))
     e("s_cbranch_scc0 %s" % lab_pstore)
-    # f32 rows (final output, or f32 partials): element (row, column) at OB + row * RSTR + column * 4.
+    # f32: final rows (row-major), or partials in layout [column / 4][row][4] (FLG bit 7: a store instruction then writes runs of 512 bytes).
+    # Element (row, column) at OB + row * RSTR + (column / 4) * CSTR, CSTR = 16 bytes or a column group's rows of a slot (OSTR).
     # acc[cb][hb] register 4 q + c of lane (rl, g) is row 32 hb + rl, column 128 w + 32 cb + 8 q + 4 g + c.
+    e("s_bitcmp1_b32 %s, 7" % s(FLG))
+    e("s_cselect_b32 %s, %s, 16" % (s(CSTR), s(OSTR)))
     e("v_mul_lo_u32 %s, %s, %s" % (v(T[0]), v(X1), s(RSTR)))
-    e("v_lshlrev_b32 %s, 4, %s" % (v(T[1]), v(X2)))
+    e("v_mul_lo_u32 %s, %s, %s" % (v(T[1]), v(X2), s(CSTR)))
     e("v_add_u32 %s, %s, %s" % (v(T[0]), v(T[0]), v(T[1])))
-    e("s_lshl_b32 %s, %s, 9" % (s(S0), s(WAVE)))
-    e("v_add_u32 %s, %s, %s" % (v(T[0]), s(S0), v(T[0])))              # rl * RSTR + 16 g + 512 w
+    e("s_lshl_b32 %s, %s, 5" % (s(S0), s(WAVE)))
+    e("s_mul_i32 %s, %s, %s" % (s(S0), s(S0), s(CSTR)))
+    e("v_add_u32 %s, %s, %s" % (v(T[0]), s(S0), v(T[0])))              # rl * RSTR + (32 w + g) * CSTR
     e("s_lshl_b32 %s, %s, 5" % (s(S1), s(RSTR)))                       # 32 rows
-    e("s_mov_b64 %s, %s" % (s(SB, 2), s(OB, 2)))
+    e("s_lshl_b32 %s, %s, 1" % (s(CSTR), s(CSTR)))                     # from one store to the next: two column groups
+    e("s_mov_b64 %s, %s" % (s(S2, 2), s(OB, 2)))
     for hb in range(nhb):
         e("s_mov_b64 exec, %s" % s(VM[hb], 2))
+        e("s_mov_b64 %s, %s" % (s(SB, 2), s(S2, 2)))
         for cb in range(4):
             for q in range(4):
                 r = S if (cb * 4 + q) % 2 == 0 else S + 4          # alternate two 4-register staging groups
@@ -1156,9 +1163,11 @@ def epilogue(nhb):
                     e("v_accvgpr_read_b32 %s, %s" % (v(r + c), a(16 * (4 * cb + hb) + 4 * q + c)))
                 for c in range(4):
                     e("v_mul_f32 %s, %s, %s" % (v(r + c), v(r + c), v(T[4 + hb])))
-                e("global_store_dwordx4 %s, %s, %s offset:%d" % (v(T[0]), v(r, 4), s(SB, 2), (32 * cb + 8 * q) * 4))
-        e("s_add_u32 %s, %s, %s" % (s(SB), s(SB), s(S1)))
-        e("s_addc_u32 %s, %s, 0" % (s(SB + 1), s(SB + 1)))
+                e("global_store_dwordx4 %s, %s, %s" % (v(T[0]), v(r, 4), s(SB, 2)))
+                e("s_add_u32 %s, %s, %s" % (s(SB), s(SB), s(CSTR)))
+                e("s_addc_u32 %s, %s, 0" % (s(SB + 1), s(SB + 1)))
+        e("s_add_u32 %s, %s, %s" % (s(S2), s(S2), s(S1)))
+        e("s_addc_u32 %s, %s, 0" % (s(S3), s(S3)))
     e("s_branch %s" % lab_sdone)
     e("%s:" % lab_pstore)
     # f16 partials O / l, layout [column / 8][row][8 halves]: the 8 bytes of lane (rl, g) for column group 16 w + 4 cb + q

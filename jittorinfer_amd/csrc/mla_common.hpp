@@ -55,7 +55,7 @@ struct KParams {
     float *         dst;
     int64_t         dst_stride;  // floats
     _Float16 *      part_o;      // split-K partials O_c / l_c as f16: [n_seq][n_splits][dv_total/8][n_rows][8], or, when
-                                 // part_f32 is set (small problems: no second rounding), as f32 rows [n_seq][n_splits][n_rows][dv_total]
+                                 // part_f32 is set (small problems: no second rounding), as f32 [n_seq][n_splits][dv_total/4][n_rows][4]
     int             part_f32;
     float *         part_ml;     // [n_seq][n_splits][n_rows][2]  (max in log2 units, sum)
     int             n_head, n_tok, n_rows;

@@ -532,9 +532,9 @@ __device__ __forceinline__ void decode_body() {
     // per-thread pointers for the wave program, handed over through LDS
     // final output: row-major dst rows.  split-K partial: [column/8][row][8] inside this (sequence, split) block.
     const int64_t pblock = (int64_t) slot * p.slot_rows * p.dv_total;  // in f16 elements
-    // (f32 partials are rows of dv_total floats: the wave program stores them the way it stores final output rows)
+    // (f32 partials: [column/4][row][4])
     void * optr = row_valid ? (direct ? (void *) (p.dst + orow * p.dst_stride + p.v_col0 + 4 * g)
-                               : p.part_f32    ? (void *) ((float *) p.part_o + prow * p.dv_total + 4 * g)
+                               : p.part_f32    ? (void *) ((float *) p.part_o + pblock + ((int64_t) g * p.slot_rows + lrow) * 4)
                                                : (void *) (p.part_o + pblock + (int64_t) lrow * 8 + 4 * g)) : nullptr;
     float * mlptr = (!direct && g == 0 && row_valid) ? p.part_ml + prow * 2 : nullptr;
     // bias builds (ALiBi slope, soft cap; ggml-cpu.c:12041-12057): the launcher has put scale / softcap into p.scale,
@@ -578,10 +578,10 @@ __device__ __forceinline__ void decode_body() {
     const int s_kve  = __builtin_amdgcn_readfirstlane(kv_end);
     const int s_npp  = __builtin_amdgcn_readfirstlane(p.n_pool_pages - 1);
     const int s_nb1  = __builtin_amdgcn_readfirstlane((int) p.kv_nb1);
-    // bit 0: f32 row store; bit 4: V starts at column 64; bit 5: none of this wave's 32 rows exists (it only moves tiles and,
+    // bit 0: f32 stores; bit 7: of partials, by column groups, not of final rows; bit 4: V starts at column 64; bit 5: none of this wave's 32 rows exists (it only moves tiles and,
     // in the Q8_0 programs, dequantizes its share of them); bit 6 (column-split programs): the Q operands wait in the tile buffers
     const int s_flg  = __builtin_amdgcn_readfirstlane((direct || p.part_f32 ? 1 : 0) | (p.v_col0 ? 16 : 0) |
-                                                      (by * 128 + wave * 32 >= p.n_rows ? 32 : 0) | (p.q_in_kernel ? 64 : 0));
+                                                      (by * 128 + wave * 32 >= p.n_rows ? 32 : 0) | (p.q_in_kernel ? 64 : 0) | (!direct && p.part_f32 ? 128 : 0));
     const int s_ntl  = __builtin_amdgcn_readfirstlane(n_tiles);
     // id of the split's first page as a scalar: the first tiles are requested before the vector load of all page ids is back
     int pg0 = 0;
@@ -593,13 +593,13 @@ __device__ __forceinline__ void decode_body() {
     const int s_ostr = __builtin_amdgcn_readfirstlane(p.slot_rows * 16);  // bytes between the partial rows of column groups c and c+1
 
     // column-split programs: every wave stores 128 columns of all 128 rows, so the output is described by scalars -- the block's
-    // first row in dst (final rows) or in its partial slot, the byte pitch of f32 rows, and the number of rows that exist
+    // first row in dst (final rows) or in its partial slot, the byte pitch of f32 rows (16 in a partial slot), and the number of rows that exist
     const int lrow0 = block_slots ? 0 : by * 128;
     const char * out_base = direct ? (const char *) (p.dst + ((int64_t) b * p.n_rows + by * 128) * p.dst_stride + p.v_col0)
-                          : p.part_f32 ? (const char *) ((float *) p.part_o + ((int64_t) slot * p.slot_rows + lrow0) * p.dv_total)
+                          : p.part_f32 ? (const char *) ((float *) p.part_o + pblock + (int64_t) lrow0 * 4)
                                        : (const char *) (p.part_o + pblock + (int64_t) lrow0 * 8);
     const char * ml_base  = direct ? nullptr : (const char *) (p.part_ml + ((int64_t) slot * p.slot_rows + lrow0) * 2);
-    const int s_rstr = __builtin_amdgcn_readfirstlane((int) ((direct ? p.dst_stride : (int64_t) p.dv_total) * 4));
+    const int s_rstr = __builtin_amdgcn_readfirstlane(direct ? (int) (p.dst_stride * 4) : 16);
     const int s_nrv  = __builtin_amdgcn_readfirstlane(min(max(p.n_rows - by * 128, 0), 128));
 
     // mask builds of the column-split programs: byte offset of this lane's first mask element (its query token's row, tokens 4g.. of a tile)

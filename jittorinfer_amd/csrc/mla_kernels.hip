@@ -391,13 +391,13 @@ __global__ void __launch_bounds__(NTHREADS) mla_attn_tile_kernel(const KParams p
         // for the combine pass, and half the bytes of f32 (the 2^-11 rounding is averaged over the splits)
         const float pinv = 1.0f / l_tot;
         if (p.part_f32) {
-            float * o = (float *) p.part_o + prow * p.dv_total + p.d_off;
+            float * o = (float *) p.part_o + pblock + (int64_t) row * 4;
 #pragma unroll
             for (int i = 0; i < NDBW; i++)
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
                     f32x4 v = { acc[i][4 * j] * pinv, acc[i][4 * j + 1] * pinv, acc[i][4 * j + 2] * pinv, acc[i][4 * j + 3] * pinv };
-                    *(f32x4 *) (o + (wd * NDBW + i) * 32 + 8 * j + 4 * g) = v;
+                    *(f32x4 *) (o + (int64_t) ((p.d_off + (wd * NDBW + i) * 32 + 8 * j + 4 * g) / 4) * p.n_rows * 4) = v;
                 }
         } else
 #pragma unroll
@@ -621,28 +621,26 @@ __global__ void __launch_bounds__(256) mla_attn_combine_wide_kernel(const KParam
     *(float2 *) out = v;
 }
 
-// The same merge over f32 partials (rows of dv_total floats; small problems).  One thread = one (row, group of 4 columns),
-// lanes along the columns of a row.  grid = (ceil(rows/2), 1, n_seq), block = 256 = 2 rows x 128 column groups (dv <= 512)
-// or (rows, 1, n_seq) with 144 active threads for dv = 576: blockDim covers one or two rows, see the launch.
-// G splits are loaded together (a split past the end is a duplicate of the last one with weight 0): small problems are
-// latency-bound, so the group should cover every split of a row in one round -- a ragged batch of short sequences has up to 32
-// one-page pieces per sequence -- without issuing many times the loads a row with two or three splits needs.
-template <int G>
-__device__ __forceinline__ void combine_f32_row(const float2 * ml, const float * po, int64_t ml_step, int64_t po_step, int nvalid, float * dst) {
-    float M = -INFINITY, L = 0.f;
-    f32x4 o = { 0.f, 0.f, 0.f, 0.f };
-    for (int c0 = 0; c0 < nvalid; c0 += G) {
+// The same merge over f32 partials ([column/4][row][4]; small problems: a chain of latencies, not bytes).  A wave covers 16 rows x 4
+// groups of 4 columns -- runs of 256 bytes per load -- and the splits of a row are one wave's (SW = 1: a block is 16 rows x 64
+// columns) or shared by the four waves of the block, which meet in LDS (SW = 4: 16 rows x 16 columns, from 9 splits per row on).
+// G splits are loaded together (a split past the end is a duplicate of the last one with weight 0): enough for one round of most
+// rows without issuing many times the loads a row with two or three splits needs.
+// grid = (ceil(rows / 16), ceil(dv / 64) or ceil(dv / 16), n_seq), block = 256.
+template <int SW, int G>
+__device__ __forceinline__ void combine_f32_walk(const float2 * ml, const float * po, int64_t ml_step, int64_t po_step, int nvalid, int c_first, float & M, float & L, f32x4 & o) {
+    for (int c0 = c_first; c0 < nvalid; c0 += SW * G) {
         float2 mlv[G];
         f32x4  xv[G];
 #pragma unroll
         for (int k = 0; k < G; k++) {
-            const int c = min(c0 + k, nvalid - 1);
+            const int c = min(c0 + SW * k, nvalid - 1);
             mlv[k] = ml[c * ml_step];
             xv[k]  = *(const f32x4 *) (po + c * po_step);
         }
         float Mg = M;
 #pragma unroll
-        for (int k = 0; k < G; k++) if (c0 + k < nvalid) Mg = fmaxf(Mg, mlv[k].x);
+        for (int k = 0; k < G; k++) if (c0 + SW * k < nvalid) Mg = fmaxf(Mg, mlv[k].x);
         if (Mg == -INFINITY) continue;  // every split so far saw only masked keys
         const float r = fast_exp2(M - Mg);  // 0 when M was -inf
         M = Mg;
@@ -650,95 +648,54 @@ __device__ __forceinline__ void combine_f32_row(const float2 * ml, const float *
         o.x *= r; o.y *= r; o.z *= r; o.w *= r;
 #pragma unroll
         for (int k = 0; k < G; k++) {
-            const float w = (c0 + k < nvalid && mlv[k].x != -INFINITY) ? mlv[k].y * fast_exp2(mlv[k].x - M) : 0.f;
+            const float w = (c0 + SW * k < nvalid && mlv[k].x != -INFINITY) ? mlv[k].y * fast_exp2(mlv[k].x - M) : 0.f;
             L += w;
             if (w == 0.f) continue;  // that split saw only masked keys (or is padding): its partial may hold anything
             o.x += xv[k].x * w; o.y += xv[k].y * w; o.z += xv[k].z * w; o.w += xv[k].w * w;
         }
     }
+}
+
+template <bool TAIL, int SW>
+__global__ void __launch_bounds__(256) mla_attn_combine_f32_kernel(const KParams p) {
+    __shared__ float red[SW == 1 ? 1 : 4][6][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int b = blockIdx.z, row = blockIdx.x * 16 + (lane & 15);
+    const int cg = (SW == 1 ? (int) blockIdx.y * 16 + wave * 4 : (int) blockIdx.y * 4) + (lane >> 4);
+    const bool store = combine_row<TAIL>(p, b, row) && cg * 4 < p.dv_total;   // (lanes without a row or a column stay for the barrier)
+    row = min(row, p.n_rows - 1);
+    const int cgc = min(cg, p.dv_total / 4 - 1);
+    const int seq_len = p.block_table ? min(p.seq_lens[b], (int) p.bt_stride * MLA_PAGE_TOKENS) : (int) p.n_kv;
+    int slot0, nvalid, lrow, slot_rows;
+    partial_slots<TAIL>(p, b, row, seq_len, slot0, nvalid, lrow, slot_rows);   // (nvalid < 0: the rows are there already)
+    const float2 * ml = (const float2 *) p.part_ml + (int64_t) slot0 * slot_rows + lrow;
+    const float *  po = (const float *) p.part_o + (int64_t) slot0 * slot_rows * p.dv_total + ((int64_t) cgc * slot_rows + lrow) * 4;
+    const int64_t ml_step = slot_rows, po_step = (int64_t) slot_rows * p.dv_total;
+    float M = -INFINITY, L = 0.f;
+    f32x4 o = { 0.f, 0.f, 0.f, 0.f };
+    const int c_first = SW == 1 ? 0 : wave;
+    if (nvalid <= 4 * SW)      combine_f32_walk<SW, 4>(ml, po, ml_step, po_step, nvalid, c_first, M, L, o);
+    else if (nvalid <= 8 * SW) combine_f32_walk<SW, 8>(ml, po, ml_step, po_step, nvalid, c_first, M, L, o);
+    else                       combine_f32_walk<SW, 16>(ml, po, ml_step, po_step, nvalid, c_first, M, L, o);
+    if constexpr (SW == 4) {
+        red[wave][0][lane] = M; red[wave][1][lane] = L;
+        red[wave][2][lane] = o.x; red[wave][3][lane] = o.y; red[wave][4][lane] = o.z; red[wave][5][lane] = o.w;
+        __syncthreads();
+        if (wave != 0) return;
+        const float Mq = fmaxf(fmaxf(red[0][0][lane], red[1][0][lane]), fmaxf(red[2][0][lane], red[3][0][lane]));
+        L = 0.f;
+        o = f32x4{ 0.f, 0.f, 0.f, 0.f };
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+            const float mw = red[w][0][lane];
+            const float rs = mw == -INFINITY ? 0.f : fast_exp2(mw - Mq);   // (a wave without a valid split adds nothing)
+            L += red[w][1][lane] * rs;
+            o.x += red[w][2][lane] * rs; o.y += red[w][3][lane] * rs; o.z += red[w][4][lane] * rs; o.w += red[w][5][lane] * rs;
+        }
+    }
+    if (!store || nvalid < 0) return;
     const float inv = 1.0f / L;  // no valid key at all: 0 * inf = NaN, like the reference
-    *(f32x4 *) dst = f32x4{ o.x * inv, o.y * inv, o.z * inv, o.w * inv };
-}
-
-template <bool TAIL>
-__global__ void __launch_bounds__(256) mla_attn_combine_f32_kernel(const KParams p, int groups_per_row) {
-    const int rows_per_block = 256 / groups_per_row;
-    int b = blockIdx.z, row = blockIdx.x * rows_per_block + threadIdx.x / groups_per_row;
-    const int cg  = threadIdx.x % groups_per_row;
-    if (!combine_row<TAIL>(p, b, row)) return;
-    const int seq_len = p.block_table ? min(p.seq_lens[b], (int) p.bt_stride * MLA_PAGE_TOKENS) : (int) p.n_kv;
-    if ((int) threadIdx.x >= rows_per_block * groups_per_row || cg * 4 >= p.dv_total) return;
-    int slot0, nvalid, lrow, slot_rows;
-    partial_slots<TAIL>(p, b, row, seq_len, slot0, nvalid, lrow, slot_rows);
-    if (nvalid < 0) return;
-    const float2 * ml = (const float2 *) p.part_ml + (int64_t) slot0 * slot_rows + lrow;
-    const float *  po = (const float *) p.part_o + ((int64_t) slot0 * slot_rows + lrow) * p.dv_total + cg * 4;
-    const int64_t ml_step = slot_rows, po_step = (int64_t) slot_rows * p.dv_total;
-    float * dst = p.dst + ((int64_t) b * p.n_rows + row) * p.dst_stride + p.v_col0 + cg * 4;
-    if (nvalid <= 4)       combine_f32_row<4>(ml, po, ml_step, po_step, nvalid, dst);
-    else if (nvalid <= 16) combine_f32_row<16>(ml, po, ml_step, po_step, nvalid, dst);
-    else                   combine_f32_row<32>(ml, po, ml_step, po_step, nvalid, dst);
-}
-
-// f32 partials, rows with more than 32 splits (a single sequence of a decode step: 64 one-page splits at 8192 keys, 256 pieces at
-// 131 072): the four waves of a block share the walk over the splits of one row -- wave w takes splits w, w + 4, ..., 16 in flight,
-// for 64 groups of 4 columns -- and meet in LDS.  grid = (rows, ceil(dv / 256), n_seq), block = 256.
-__global__ void __launch_bounds__(256) mla_attn_combine_f32_wide_kernel(const KParams p) {
-    __shared__ float red[4][6][64];
-    constexpr int G = 16;
-    const int b = blockIdx.z, row = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int cg = min((int) blockIdx.y * 64 + lane, p.dv_total / 4 - 1);   // (lanes past the row's end repeat its last group and store nothing)
-    const int seq_len = p.block_table ? min(p.seq_lens[b], (int) p.bt_stride * MLA_PAGE_TOKENS) : (int) p.n_kv;
-    int slot0, nvalid, lrow, slot_rows;
-    partial_slots(p, b, row, seq_len, slot0, nvalid, lrow, slot_rows);
-    if (nvalid < 0) return;   // (uniform over the block: one row)
-    const float2 * ml = (const float2 *) p.part_ml + (int64_t) slot0 * slot_rows + lrow;
-    const float *  po = (const float *) p.part_o + ((int64_t) slot0 * slot_rows + lrow) * p.dv_total + cg * 4;
-    const int64_t ml_step = slot_rows, po_step = (int64_t) slot_rows * p.dv_total;
-    float M = -INFINITY, L = 0.f;
-    f32x4 o = { 0.f, 0.f, 0.f, 0.f };
-    for (int c0 = wave; c0 < nvalid; c0 += 4 * G) {
-        float2 mlv[G];
-        f32x4  xv[G];
-#pragma unroll
-        for (int k = 0; k < G; k++) {
-            const int c = min(c0 + 4 * k, nvalid - 1);
-            mlv[k] = ml[c * ml_step];
-            xv[k]  = *(const f32x4 *) (po + c * po_step);
-        }
-        float Mg = M;
-#pragma unroll
-        for (int k = 0; k < G; k++) if (c0 + 4 * k < nvalid) Mg = fmaxf(Mg, mlv[k].x);
-        if (Mg == -INFINITY) continue;  // every split so far saw only masked keys
-        const float r = fast_exp2(M - Mg);  // 0 when M was -inf
-        M = Mg;
-        L *= r;
-        o.x *= r; o.y *= r; o.z *= r; o.w *= r;
-#pragma unroll
-        for (int k = 0; k < G; k++) {
-            const float w = (c0 + 4 * k < nvalid && mlv[k].x != -INFINITY) ? mlv[k].y * fast_exp2(mlv[k].x - M) : 0.f;
-            L += w;
-            if (w == 0.f) continue;  // that split saw only masked keys (or is padding): its partial may hold anything
-            o.x += xv[k].x * w; o.y += xv[k].y * w; o.z += xv[k].z * w; o.w += xv[k].w * w;
-        }
-    }
-    red[wave][0][lane] = M; red[wave][1][lane] = L;
-    red[wave][2][lane] = o.x; red[wave][3][lane] = o.y; red[wave][4][lane] = o.z; red[wave][5][lane] = o.w;
-    __syncthreads();
-    if (wave != 0 || (int) blockIdx.y * 64 + lane >= p.dv_total / 4) return;
-    float Mq = fmaxf(fmaxf(red[0][0][lane], red[1][0][lane]), fmaxf(red[2][0][lane], red[3][0][lane]));
-    float Lq = 0.f;
-    f32x4 oq = { 0.f, 0.f, 0.f, 0.f };
-#pragma unroll
-    for (int w = 0; w < 4; w++) {
-        const float mw = red[w][0][lane];
-        const float rs = mw == -INFINITY ? 0.f : fast_exp2(mw - Mq);   // (a wave without a valid split adds nothing)
-        Lq += red[w][1][lane] * rs;
-        oq.x += red[w][2][lane] * rs; oq.y += red[w][3][lane] * rs; oq.z += red[w][4][lane] * rs; oq.w += red[w][5][lane] * rs;
-    }
-    const float inv = 1.0f / Lq;  // no valid key at all: 0 * inf = NaN, like the reference
-    float * dst = p.dst + ((int64_t) b * p.n_rows + row) * p.dst_stride + p.v_col0 + cg * 4;
-    *(f32x4 *) dst = f32x4{ oq.x * inv, oq.y * inv, oq.z * inv, oq.w * inv };
+    *(f32x4 *) (p.dst + ((int64_t) b * p.n_rows + row) * p.dst_stride + p.v_col0 + cg * 4) = f32x4{ o.x * inv, o.y * inv, o.z * inv, o.w * inv };
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -1320,16 +1277,11 @@ static int launch_phases(const mla_attn_args * a, void * stream, int phases) {
     auto combine = [&](int dv) -> int {
         const unsigned c_rows = pl.tail_splits ? (unsigned) n_tail * 128 : (unsigned) kp.n_rows, c_seq = pl.tail_splits ? 1 : (unsigned) a->n_seq;
         const int splits_per_row = pl.tail_splits ? pl.tail_splits : pl.balanced ? (pl.n_wg + pl.n_units - 1) / pl.n_units : pl.n_splits;
-        if (pl.part_f32 && splits_per_row > 32) {   // (one or two sequences: the waves of a block share the walk over a row's splits)
-            dim3 gw((unsigned) kp.n_rows, (unsigned) ((dv / 4 + 63) / 64), (unsigned) a->n_seq);
-            hipLaunchKernelGGL(mla_attn_combine_f32_wide_kernel, gw, dim3(256), 0, st, kp);
-            return (int) hipGetLastError();
-        }
         if (pl.part_f32) {
-            const int groups = dv / 4, rows_per_block = 256 / groups;   // 128 -> 2 rows, 144 -> 1 row
-            dim3 g((c_rows + rows_per_block - 1) / rows_per_block, 1, c_seq);
-            auto kern = pl.tail_splits ? mla_attn_combine_f32_kernel<true> : mla_attn_combine_f32_kernel<false>;
-            hipLaunchKernelGGL(kern, g, dim3(256), 0, st, kp, groups);
+            const bool share = splits_per_row > 8;
+            dim3 g((c_rows + 15) / 16, (unsigned) (share ? (dv + 15) / 16 : (dv + 63) / 64), c_seq);
+            auto kern = pl.tail_splits ? mla_attn_combine_f32_kernel<true, 1> : share ? mla_attn_combine_f32_kernel<false, 4> : mla_attn_combine_f32_kernel<false, 1>;   // (a tail has at most 8 splits per row)
+            hipLaunchKernelGGL(kern, g, dim3(256), 0, st, kp);
             return (int) hipGetLastError();
         }
         // rows with many splits (few long sequences): four lanes share the walk over a row's splits
