@@ -59,6 +59,8 @@ struct KParams {
     int             part_f32;
     float *         part_ml;     // [n_seq][n_splits][n_rows][2]  (max in log2 units, sum)
     int             n_head, n_tok, n_rows;
+    int             seq_shift;     // a decode step whose heads are taken in 2^seq_shift groups: "sequence" b of the launch is group b % 2^seq_shift
+                                   // of sequence b >> seq_shift (n_head is a group's, the rows of dst are the same either way)
     int             n_splits, split_tokens;
     int             dv_total, d_off;
     float           scale, softcap, max_bias, m0, m1;
@@ -102,6 +104,11 @@ struct KParams {
                                    //   (nullptr: its program rounds Q itself), and the rounding it wants (1: f16, 2: bf16 written as f16)
     int             tok_mode;
 };
+
+// Where Q of "sequence" b of a launch starts (q_nb3: from one sequence to the next; shift: seq_shift, or 0 where the launch has no groups).
+template <typename KP> __device__ __forceinline__ int64_t q_seq_offset(const KP & p, int b, int64_t q_nb3, int shift) {
+    return (int64_t) (b >> shift) * q_nb3 + (int64_t) (b & ((1 << shift) - 1)) * p.n_head * p.q_nb2;
+}
 
 template <typename T, typename U> __device__ __forceinline__ T bitcast(U u) { return __builtin_bit_cast(T, u); }
 

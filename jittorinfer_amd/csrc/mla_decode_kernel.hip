@@ -157,7 +157,7 @@ __device__ __forceinline__ void sched_scan(int * S, int count, int base, int n_u
 
 // The first piece of workgroup v: {item, kv_begin, kv_end, id of its first page (paged), whole item?, list position after
 // the piece, end of the run, sequence length}; kv_begin >= kv_end: the workgroup has no work.
-template <typename KP> __device__ __forceinline__ void sched_first_piece(const KP & p, const int * S, int v, int unit_tokens, int hdr[8]) {
+template <typename KP> __device__ __forceinline__ void sched_first_piece(const KP & p, const int * S, int v, int unit_tokens, int hdr[8], int seq_shift) {
     const int total = S[p.n_units], quota = (total + p.n_wg - 1) / p.n_wg;
     const int pos = min(v * quota, total), end = min(pos + quota, total);
     hdr[0] = hdr[1] = hdr[2] = hdr[3] = hdr[4] = hdr[7] = 0;
@@ -171,9 +171,9 @@ template <typename KP> __device__ __forceinline__ void sched_first_piece(const K
     hdr[1] = base + (pos - first) * unit_tokens;
     hdr[2] = base + (piece_end - first) * unit_tokens;
     if (p.balanced == 1) {
-        const int len = min(p.seq_lens[it], p.key_cap);
+        const int len = min(p.seq_lens[it >> seq_shift], p.key_cap);
         hdr[2] = min(len, hdr[2]);
-        hdr[3] = min(max(p.block_table[(int64_t) it * p.bt_stride + (pos - first)], 0), p.n_pool_pages - 1);
+        hdr[3] = min(max(p.block_table[(int64_t) (it >> seq_shift) * p.bt_stride + (pos - first)], 0), p.n_pool_pages - 1);
         hdr[7] = len;
     } else {
         hdr[7] = p.key_cap;
@@ -206,13 +206,13 @@ __device__ __forceinline__ void sched_prefix(const KParams & p) {
     __shared__ int S[2 * SCHED_MAX_SEQ + 8];
     const int t = threadIdx.x;
     int pages = 0;
-    if (t < p.n_units) pages = (max(min(p.seq_lens[t], p.key_cap), 0) + MLA_PAGE_TOKENS - 1) / MLA_PAGE_TOKENS;
+    if (t < p.n_units) pages = (max(min(p.seq_lens[t >> p.seq_shift], p.key_cap), 0) + MLA_PAGE_TOKENS - 1) / MLA_PAGE_TOKENS;
     sched_scan(S, pages, 0, p.n_units);
     if (t <= p.n_units) p.sched[t] = S[t];
     if (t == 0 && p.n_units == SCHED_MAX_SEQ) p.sched[SCHED_MAX_SEQ] = S[SCHED_MAX_SEQ];
     if (t >= p.n_wg) return;
     int hdr[8];
-    sched_first_piece(p, S, t, MLA_PAGE_TOKENS, hdr);
+    sched_first_piece(p, S, t, MLA_PAGE_TOKENS, hdr, p.seq_shift);
     for (int i = 0; i < 8; i++) p.wg_first[8 * t + i] = hdr[i];
 }
 
@@ -235,15 +235,15 @@ template <bool F16> __device__ __forceinline__ u32x2 round4(const f32x4 x) {
 }
 // Lane r < 32 works out where row row0 + r of Q starts (rows past n_rows: the last one) and leaves the address of its byte col0 in
 // this wave's table of 32 entries in LDS.
-template <typename KP> __device__ __forceinline__ void q_row_table(const KP & p, int b, int row0, int col0, unsigned long long * rowptr, int lane) {
+template <typename KP> __device__ __forceinline__ void q_row_table(const KP & p, int b, int row0, int col0, unsigned long long * rowptr, int lane, int seq_shift) {
     const int row = min(row0 + (lane & 31), p.n_rows - 1), tq = row / p.n_head, head = row - tq * p.n_head;
-    if (lane < 32) rowptr[lane] = (unsigned long long) (p.q + (int64_t) b * p.q_nb3 + (int64_t) tq * p.q_nb1 + (int64_t) head * p.q_nb2 + col0);
+    if (lane < 32) rowptr[lane] = (unsigned long long) (p.q + q_seq_offset(p, b, p.q_nb3, seq_shift) + (int64_t) tq * p.q_nb1 + (int64_t) head * p.q_nb2 + col0);
 }
 template <bool F16, int NROW, int C4, typename KP>
 __device__ __forceinline__ void stage_q_rows(const KP & p, int b, int row0, int col0, unsigned char * lds, unsigned long long * rowptr, int lane) {
     constexpr int NLD = (C4 + 63) / 64;   // loads per row; in the last one the lanes past the end of the row repeat its last group
     constexpr int GRP = 8, NG = NROW / GRP;   // rows per group; the loads of the next group are issued ahead of the work on this one
-    q_row_table(p, b, row0, col0, rowptr, lane);   // the loop below is straight-line code with scalar row addresses
+    q_row_table(p, b, row0, col0, rowptr, lane, 0);   // the loop below is straight-line code with scalar row addresses
     const int lane_last = min(lane, C4 - 64 * (NLD - 1) - 1);
     f32x4 x[2][GRP][NLD];
     auto load = [&](int g) {
@@ -288,12 +288,15 @@ __device__ __forceinline__ void stage_q_rows(const KP & p, int b, int row0, int 
 typedef const __attribute__((address_space(4))) KParams KParamsArg;
 // STREAM (masked column-split and k-split programs): the build whose tile copies carry the non-temporal hint
 // RSBIAS (masked row-split programs of the f16 kinds: SRC_F16, SRC_BF16_CVT, SRC_Q8): the build with ALiBi slope and soft cap
+// GROUPS: the heads of a sequence are taken in 2^p.seq_shift groups, each a "sequence" of the launch (unmasked k-split programs and those
+// for two row blocks)
 // TAIL: the launch has a tail of row blocks that several workgroups share (p.tail_splits)
-template <int KVT, bool MASK, int KOFF, bool OPAQUE, bool STREAM = false, bool RSBIAS = false, bool TAIL = false>
+template <int KVT, bool MASK, int KOFF, bool OPAQUE, bool STREAM = false, bool RSBIAS = false, bool TAIL = false, bool GROUPS = false>
 __device__ __forceinline__ void decode_body() {
     static_assert(!RSBIAS || (MASK && (KVT == SRC_F16 || KVT == SRC_BF16_CVT || KVT == SRC_Q8)), "bias builds of the row-split programs");
     KParamsArg * p_ptr = (KParamsArg *) ((const __attribute__((address_space(4))) char *) __builtin_amdgcn_kernarg_segment_ptr() + KOFF);
     KParamsArg & p = *p_ptr;
+    const int seq_shift = GROUPS ? p.seq_shift : 0;
     constexpr int HANDOFF_OFF = handoff_off(KVT);
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
 
@@ -401,7 +404,7 @@ __device__ __forceinline__ void decode_body() {
             __syncthreads();   // (W is read; the tile buffers may be written)
         } else {
             int hdr[8];
-            sched_first_piece(p, sched, bx, TILE_TOK, hdr);
+            sched_first_piece(p, sched, bx, TILE_TOK, hdr, 0);
             for (int i = 0; i < 8; i++) first_piece[i] = __builtin_amdgcn_readfirstlane(hdr[i]);
             if (first_piece[1] >= first_piece[2]) return;
             run_pos = first_piece[5]; run_end = first_piece[6]; run_item = first_piece[0] + 1;
@@ -413,7 +416,7 @@ __device__ __forceinline__ void decode_body() {
         const int t = threadIdx.x;
         int pages = 0, len = 0;
         if (t < p.n_units) {
-            len   = p.seq_lens[t];
+            len   = p.seq_lens[t >> seq_shift];
             pages = (max(min(len, p.key_cap), 0) + MLA_PAGE_TOKENS - 1) / MLA_PAGE_TOKENS;
         }
         sched_scan(sched, pages, len, p.n_units);
@@ -422,7 +425,7 @@ __device__ __forceinline__ void decode_body() {
             if (t == 0 && p.n_units == SCHED_MAX_SEQ) p.sched[SCHED_MAX_SEQ] = sched[SCHED_MAX_SEQ];
         }
         int hdr[8];
-        sched_first_piece(p, sched, bx, MLA_PAGE_TOKENS, hdr);
+        sched_first_piece(p, sched, bx, MLA_PAGE_TOKENS, hdr, seq_shift);
         for (int i = 0; i < 8; i++) first_piece[i] = __builtin_amdgcn_readfirstlane(hdr[i]);
         if (first_piece[1] >= first_piece[2]) return;
         run_pos = first_piece[5]; run_end = first_piece[6]; run_item = first_piece[0] + 1;
@@ -433,7 +436,7 @@ __device__ __forceinline__ void decode_body() {
         if (first_piece[1] >= first_piece[2]) return;
         for (int i = threadIdx.x; i <= p.n_units; i += NTHREADS) {
             sched[i] = p.sched[i];
-            if (i < p.n_units) sched[SCHED_MAX_SEQ + 8 + i] = p.seq_lens[i];
+            if (i < p.n_units) sched[SCHED_MAX_SEQ + 8 + i] = p.seq_lens[i >> seq_shift];
         }
         run_pos = first_piece[5]; run_end = first_piece[6]; run_item = first_piece[0] + 1;
     }
@@ -481,7 +484,7 @@ __device__ __forceinline__ void decode_body() {
         slot  = bx + item;
         split = 1;   // not the first split of anything: an empty piece writes nothing
     } else {
-        seq_len  = p.block_table ? min(p.seq_lens[b], p.key_cap) : p.key_cap;
+        seq_len  = p.block_table ? min(p.seq_lens[b >> seq_shift], p.key_cap) : p.key_cap;
         kv_begin = split * p.split_tokens;
         kv_end   = min(seq_len, kv_begin + p.split_tokens);
         slot     = tail ? (int) blockIdx.x - p.tail_first : b * p.n_splits + split;
@@ -565,13 +568,13 @@ __device__ __forceinline__ void decode_body() {
     if constexpr (KVT == SRC_BF16_CSQ || KVT == SRC_F16_CSQ) {
         stage_q_rows<KVT == SRC_F16_CSQ, 32, 144>(p, b, by * 128 + wave * 32, 0, smem + wave * TILE_BYTES, q_rows, lane);
     } else if constexpr (is_ks(KVT)) {
-        q_row_table(p, b, 0, wave * 576, q_rows, lane);
+        q_row_table(p, b, 0, wave * 576, q_rows, lane, seq_shift);
     }
     // this wave's packed Q operands: [seq][row block][wave][k-step][lane][16 bytes], written by mla_q_pack_kernel (the programs
     // that take Q from LDS get no image)
     const char * qpack = (const char *) p.q_pack + ((((int64_t) b * ((p.n_rows + 127) / 128) + by) * 4) * KSTEPS) * 1024;  // + wave*36 KB, added in the wave program
-    const char *    kv_base = p.kv + (p.block_table ? 0 : (int64_t) b * p.kv_nb3);
-    const int32_t * bt_row  = p.block_table ? p.block_table + (int64_t) b * p.bt_stride : nullptr;
+    const char *    kv_base = p.kv + (p.block_table ? 0 : (int64_t) (b >> seq_shift) * p.kv_nb3);
+    const int32_t * bt_row  = p.block_table ? p.block_table + (int64_t) (b >> seq_shift) * p.bt_stride : nullptr;
     // uniform scalars, forced into SGPRs
     const int c_log2_bits = p.c_log2_bits;
     const int s_kvb  = __builtin_amdgcn_readfirstlane(kv_begin);
@@ -728,8 +731,8 @@ __device__ __forceinline__ void decode_body() {
   }
 }
 
-template <int KVT, bool MASK, bool STREAM = false, bool RSBIAS = false, bool TAIL = false>
-__global__ void __launch_bounds__(NTHREADS) mla_decode_kernel(const KParams) { decode_body<KVT, MASK, 0, false, STREAM, RSBIAS, TAIL>(); }   // (the body reads the argument segment)
+template <int KVT, bool MASK, bool STREAM = false, bool RSBIAS = false, bool TAIL = false, bool GROUPS = false>
+__global__ void __launch_bounds__(NTHREADS) mla_decode_kernel(const KParams) { decode_body<KVT, MASK, 0, false, STREAM, RSBIAS, TAIL, GROUPS>(); }   // (the body reads the argument segment)
 
 // A masked launch of few heads issued in two forms (the launcher's comment tells why): pb describes it as row blocks of 128 rows
 // (balanced == 2), pt token by token (balanced == 3: every query token a sequence of one token, its mask row that sequence's
@@ -1010,7 +1013,7 @@ __global__ void __launch_bounds__(NTHREADS) mla_q_pack_kernel(const KParams p) {
     if (w.n_rows <= 128 && w.wave * 32 >= w.n_rows) return;   // a wave of the decode kernel without a row that computes nothing: its image is never used
     const int row = min(w.rb * 128 + w.wave * 32 + rl, w.n_rows - 1);
     const int tq = row / p.n_head, head = row - tq * p.n_head;
-    const float * qrow = (const float *) (p.q + (int64_t) tq * p.q_nb1 + (int64_t) head * p.q_nb2 + (int64_t) w.b * w.q_nb3) + 8 * g;
+    const float * qrow = (const float *) (p.q + (int64_t) tq * p.q_nb1 + (int64_t) head * p.q_nb2 + q_seq_offset(p, w.b, w.q_nb3, p.seq_shift)) + 8 * g;
     u32x4 * out = (u32x4 *) w.image + ((((int64_t) w.b * w.n_rb + w.rb) * 4 + w.wave) * KSTEPS) * 64 + lane;
     const f32x4 x0 = *(const f32x4 *) (qrow + 16 * ks);
     const f32x4 x1 = *(const f32x4 *) (qrow + 16 * ks + 4);
@@ -1041,7 +1044,7 @@ __global__ void __launch_bounds__(NTHREADS) mla_q_pack_q8_kernel(const KParams p
     // waves without a row too; the token form leaves such a wave's part as it is -- its values are never used)
     const int row = min(w.rb * 128 + w.wave * 32 + rl, w.n_rows - 1);
     const int tq = row / p.n_head, head = row - tq * p.n_head;
-    const float * qrow = (const float *) (p.q + (int64_t) tq * p.q_nb1 + (int64_t) head * p.q_nb2 + (int64_t) w.b * w.q_nb3);
+    const float * qrow = (const float *) (p.q + (int64_t) tq * p.q_nb1 + (int64_t) head * p.q_nb2 + q_seq_offset(p, w.b, w.q_nb3, p.seq_shift));
     u32x4 * out = (u32x4 *) w.image + ((((int64_t) w.b * w.n_rb + w.rb) * 4 + w.wave) * KSTEPS) * 64 + lane;
     f32x4 x[4];
     x[0] = *(const f32x4 *) (qrow + 32 * j + 8 * g);
@@ -1152,12 +1155,12 @@ hipError_t launch_q8_to_f16(const char * src, int64_t src_nb1, int64_t src_nb3, 
     return hipGetLastError();
 }
 
-template <int KVT, bool MASK, bool STREAM = false, bool RSBIAS = false, bool TAIL = false>
+template <int KVT, bool MASK, bool STREAM = false, bool RSBIAS = false, bool TAIL = false, bool GROUPS = false>
 static hipError_t launch_variant(const KParams & kp, dim3 grid, hipStream_t st) {
     static bool attr_done[MLA_MAX_DEVICES];
-    const hipError_t e = raise_lds_limit((const void *) mla_decode_kernel<KVT, MASK, STREAM, RSBIAS, TAIL>, attr_done);
+    const hipError_t e = raise_lds_limit((const void *) mla_decode_kernel<KVT, MASK, STREAM, RSBIAS, TAIL, GROUPS>, attr_done);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((mla_decode_kernel<KVT, MASK, STREAM, RSBIAS, TAIL>), grid, dim3(NTHREADS), (size_t) lds_total(KVT), st, kp);
+    hipLaunchKernelGGL((mla_decode_kernel<KVT, MASK, STREAM, RSBIAS, TAIL, GROUPS>), grid, dim3(NTHREADS), (size_t) lds_total(KVT), st, kp);
     return hipGetLastError();
 }
 
@@ -1303,6 +1306,11 @@ hipError_t launch_decode_fast(const KParams & kp_in, int kv_type, dim3 grid, hip
     if (kv_type == MLA_TYPE_Q8_0) return m ? launch_variant<SRC_Q8, true>(kp, grid, st) : launch_variant<SRC_Q8, false>(kp, grid, st);
     if (ks && m && stream) return kv_type == MLA_TYPE_F16 ? launch_variant<SRC_F16_KS, true, true>(kp, grid, st) : launch_variant<SRC_BF16_KS, true, true>(kp, grid, st);
     if (ks && m) return kv_type == MLA_TYPE_F16 ? launch_variant<SRC_F16_KS, true>(kp, grid, st) : launch_variant<SRC_BF16_KS, true>(kp, grid, st);
+    if (kp.seq_shift) {
+        if (m || !(ks || csh)) return hipErrorInvalidValue;   // (make_plan groups no others)
+        if (ks) return kv_type == MLA_TYPE_F16 ? launch_variant<SRC_F16_KS, false, false, false, false, true>(kp, grid, st) : launch_variant<SRC_BF16_KS, false, false, false, false, true>(kp, grid, st);
+        return kv_type == MLA_TYPE_F16 ? launch_variant<SRC_F16_CSH, false, false, false, false, true>(kp, grid, st) : launch_variant<SRC_BF16_CSH, false, false, false, false, true>(kp, grid, st);
+    }
     if (ks) return kv_type == MLA_TYPE_F16 ? launch_variant<SRC_F16_KS, false>(kp, grid, st) : launch_variant<SRC_BF16_KS, false>(kp, grid, st);
     if (csh) return kv_type == MLA_TYPE_F16 ? launch_variant<SRC_F16_CSH, false>(kp, grid, st) : launch_variant<SRC_BF16_CSH, false>(kp, grid, st);
     if (cs && q_in_kernel && kv_type == MLA_TYPE_F16) return m ? launch_variant<SRC_F16_CSQ, true>(kp, grid, st) : launch_variant<SRC_F16_CSQ, false>(kp, grid, st);

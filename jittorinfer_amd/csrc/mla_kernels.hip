@@ -480,7 +480,7 @@ __global__ void __launch_bounds__(256) mla_attn_combine_kernel(const KParams p) 
     int b = blockIdx.z, row = blockIdx.x * 16 + (threadIdx.x & 15);
     const int cg  = blockIdx.y * 32 + (threadIdx.x >> 4);
     if (!combine_row<TAIL>(p, b, row) || cg * 8 >= p.dv_total) return;
-    const int seq_len = p.block_table ? min(p.seq_lens[b], (int) p.bt_stride * MLA_PAGE_TOKENS) : (int) p.n_kv;
+    const int seq_len = p.block_table ? min(p.seq_lens[b >> p.seq_shift], (int) p.bt_stride * MLA_PAGE_TOKENS) : (int) p.n_kv;
     const bool two = (cg + 16) * 8 < p.dv_total;   // the second column group exists
     int slot0, nvalid, lrow, slot_rows;
     partial_slots<TAIL>(p, b, row, seq_len, slot0, nvalid, lrow, slot_rows);
@@ -581,7 +581,7 @@ __global__ void __launch_bounds__(256) mla_attn_combine_wide_kernel(const KParam
     const int sl = lane % SL;
     const int row = blockIdx.x * (64 / SL) + lane / SL;
     const int cg  = blockIdx.y * 4 + wave;
-    const int seq_len = p.block_table ? min(p.seq_lens[b], (int) p.bt_stride * MLA_PAGE_TOKENS) : (int) p.n_kv;
+    const int seq_len = p.block_table ? min(p.seq_lens[b >> p.seq_shift], (int) p.bt_stride * MLA_PAGE_TOKENS) : (int) p.n_kv;
     // (rows past the end keep their lanes: the shuffles below want whole groups; they work on the last row and store nothing)
     const int rrow = min(row, p.n_rows - 1);
     if (cg * 8 >= p.dv_total) return;
@@ -665,7 +665,7 @@ __global__ void __launch_bounds__(256) mla_attn_combine_f32_kernel(const KParams
     const bool store = combine_row<TAIL>(p, b, row) && cg * 4 < p.dv_total;   // (lanes without a row or a column stay for the barrier)
     row = min(row, p.n_rows - 1);
     const int cgc = min(cg, p.dv_total / 4 - 1);
-    const int seq_len = p.block_table ? min(p.seq_lens[b], (int) p.bt_stride * MLA_PAGE_TOKENS) : (int) p.n_kv;
+    const int seq_len = p.block_table ? min(p.seq_lens[b >> p.seq_shift], (int) p.bt_stride * MLA_PAGE_TOKENS) : (int) p.n_kv;
     int slot0, nvalid, lrow, slot_rows;
     partial_slots<TAIL>(p, b, row, seq_len, slot0, nvalid, lrow, slot_rows);   // (nvalid < 0: the rows are there already)
     const float2 * ml = (const float2 *) p.part_ml + (int64_t) slot0 * slot_rows + lrow;
@@ -908,6 +908,7 @@ struct Plan {
     int    balanced, n_wg, n_units;   // balanced schedule of the pipelined kernel (1: ragged paged decode, 2: masked launch)
     int    dual;                      // the masked launch is issued in two forms, see token_form_candidate
     int    tail_first, tail_splits;   // masked launch beyond whole rounds of workgroups: see masked_splits
+    int    seq_shift;                 // heads in 2^seq_shift groups, each a "sequence" of the launch: see head_groups
     int    seq_sorted;                // paged decode of more than 256 sequences: workgroups take the sequences longest first
 };
 
@@ -989,9 +990,44 @@ static bool masked_worth_dealing(int64_t n_items, int64_t n_tiles) {
     return n_items <= 8 ? n_tiles > 4 : n_tiles * (1280 - 6 * n_items) > 15360;   // (2 x 10 35.1 / 25.2, 4 x 5 28.1 / 24.9, 8 x 6 29.6 / 28.2, 16 x 8 33.3 / 33.9)
 }
 
+// A decode step of more than 32 heads over few keys: what a workgroup of 128 rows spends beside its tiles (147 KB of Q in, 128
+// partial rows out and merged) outweighs them, and splitting the keys further only makes more of both.  Splitting the heads makes less:
+// in groups of 32 (the k-split program, no pass that packs Q) or 64 (the program for two row blocks), each group a sequence of its own
+// on the same keys, which it reads again -- from the L2s, that few keys.  One box, bf16, 128 heads whole / in 2 / in 4 groups, us (tiles =
+// sequences x 32-key tiles): 1 x 1200 keys 22.0 / 20.0 / 17.2, 16 x 300 30.2 / 28.4 / 24.1 (160 tiles), 1 x 8192 34.6 / 28.3 / 28.2 (256), 8 x 1200
+// 36.9 / 29.1 / 30.2 (304), 2 x 8192 42.4 / 31.8 / 33.6 (512), 16 x 1200 36.1 / 32.7 / 39.8 (608), 32 x 600 33.5 / 37.8 / 43.1 (608), 4 x 8192 43.4 /
+// 36.2 / 44.1 (1024), 16 x 2400 45.7 / 43.1 / 52.6 (1200), 32 x 1200 41.9 / 42.6 (1216), 8 x 8192 52.7 / 46.1 (2048), 16 x 4800 51.5 / 55.9 (2400).
+// So: groups of 32 up to 240 tiles, groups of 64 up to 2048 while tiles x sequences <= 16000.  64 heads: groups of 32 up to 480 tiles.
+int head_groups_shift(const mla_attn_args * a) {
+    if (a->mask || a->n_tok != 1 || a->n_head <= 32 || a->n_head > 128 || a->n_splits != 0 || a->rows_per_wg != 0) return 0;
+    if (a->kv_type == MLA_TYPE_Q8_0 || (a->flags & (MLA_FLAG_F16_ACC_STRICT | MLA_FLAG_BF16_DIRECT)) || !decode_fast_applicable(a)) return 0;
+    const int64_t tiles = a->n_seq * ((key_capacity(a) + TILE_TOK - 1) / TILE_TOK);
+    const int to32 = a->n_head <= 64 ? 1 : 2;
+    if (a->n_head % (1 << to32) == 0 && a->n_seq <= 256 >> to32 && tiles <= (a->n_head <= 64 ? 480 : 240)) return to32;
+    return a->n_head > 64 && a->n_head % 2 == 0 && a->n_seq <= 128 && tiles <= 2048 && tiles * a->n_seq <= 16000 ? 1 : 0;
+}
+
+// all_rows: of a sequence of the caller's (a may be the launch as the groups of heads make it)
+static int plan_rows(const mla_attn_args * a, Plan * pl, int64_t all_rows);
+
+// The launch's own shape: the caller's, or with every group of heads a sequence.
+static mla_attn_args grouped(const mla_attn_args * a, int shift) {
+    mla_attn_args g = *a;
+    g.n_seq <<= shift; g.n_head >>= shift;
+    return g;
+}
+
 int make_plan(const mla_attn_args * a, Plan * pl) {
     const int rc = validate(a);
     if (rc) return rc;
+    const int shift = head_groups_shift(a);
+    const mla_attn_args g = grouped(a, shift);
+    const int rc2 = plan_rows(&g, pl, (int64_t) a->n_tok * a->n_head);
+    pl->seq_shift = shift;
+    return rc2;
+}
+
+static int plan_rows(const mla_attn_args * a, Plan * pl, int64_t all_rows) {
     const int64_t n_rows  = (int64_t) a->n_tok * a->n_head;
     int64_t max_len = a->block_table ? a->bt_stride * MLA_PAGE_TOKENS : a->n_kv;
     *pl = Plan{};
@@ -1060,7 +1096,7 @@ int make_plan(const mla_attn_args * a, Plan * pl) {
     // combine pass loses more than the kernel gains (16 heads x 8192 keys in 256 splits: 17.5 -> 21.3 us).
     if (pl->variant == 2 && a->n_splits == 0 && pages_per_split == 1 && !a->mask && a->kv_type != MLA_TYPE_Q8_0) {
         const int64_t n_tiles = (max_len + TILE_TOK - 1) / TILE_TOK, wgs = (int64_t) a->n_seq * pl->n_row_blocks;
-        const int64_t lim = (int64_t) (n_rows <= 32 ? 4 : 1) << 20;
+        const int64_t lim = (int64_t) (all_rows <= 32 ? 4 : 1) << 20;
         const int64_t want = std::min<int64_t>({ n_tiles, 256 / wgs, lim / ((int64_t) a->n_seq * n_rows * 512 * 4) });
         if (want > pl->n_splits) {
             const int64_t tiles_per_split = (n_tiles + want - 1) / want;
@@ -1168,7 +1204,7 @@ int mla_attn_plan(const mla_attn_args * args, mla_attn_plan_info * out) {
     const int rc = make_plan(args, &pl);
     if (rc) return rc;
     if (!out) return MLA_ERR_NULL;
-    const int a_n_seq = args->n_seq;
+    const int a_n_seq = args->n_seq << pl.seq_shift;
     out->variant      = pl.variant;
     out->rows_per_wg  = pl.rblk;
     out->n_row_blocks = pl.n_row_blocks;
@@ -1184,10 +1220,11 @@ int mla_attn_plan(const mla_attn_args * args, mla_attn_plan_info * out) {
 
 // phases: bit 0 = the attention kernels (partials or final output), bit 1 = the combine pass,
 // bit 2 = the small passes ahead of the pipelined kernel (Q operand image, key extent of the mask)
-static int launch_phases(const mla_attn_args * a, void * stream, int phases) {
+static int launch_phases(const mla_attn_args * args, void * stream, int phases) {
     Plan pl;
-    const int rc = make_plan(a, &pl);
+    const int rc = make_plan(args, &pl);
     if (rc) return rc;
+    const mla_attn_args launch = grouped(args, pl.seq_shift), * a = &launch;
     const size_t need = plan_ws(pl);
     if (need > 0 && (!a->workspace || a->workspace_size < need || ((uintptr_t) a->workspace & 255))) return MLA_ERR_WORKSPACE;
     hipStream_t st = (hipStream_t) stream;
@@ -1198,6 +1235,7 @@ static int launch_phases(const mla_attn_args * a, void * stream, int phases) {
     kp.mask = (const char *) a->mask; kp.mask_nb1 = a->mask_nb1; kp.mask_ne0 = a->mask_ne0; kp.mask_nb3 = 0;   // (shared by the sequences, ggml-cpu.c:12024)
     kp.block_table = a->block_table; kp.bt_stride = a->bt_stride; kp.seq_lens = a->seq_lens;
     kp.dst = a->dst; kp.dst_stride = a->dst_nb1 / 4;
+    kp.seq_shift = pl.seq_shift;
     kp.n_head = a->n_head; kp.n_tok = a->n_tok; kp.n_rows = a->n_tok * a->n_head;
     kp.n_splits = pl.n_splits; kp.split_tokens = pl.split_tokens;
     kp.dv_total = a->dv;

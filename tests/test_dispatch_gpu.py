@@ -84,3 +84,43 @@ def test_row_blocks_left_over_from_whole_rounds_are_split(gpu, k_type, n_seq, n_
             want = (O.flash_attn_ext_f64 if k_type == O.TYPE_F16 else O.flash_attn_ext)(
                 q[b:b + 1, :, t:t + 1], seqs[b][None, :width], k_type, dv=dv, mask=np.ascontiguousarray(mask[t:t + 1, :len(seqs[b])]), scale=U.SCALE)
             print(b, t, U.check(got[b:b + 1, t:t + 1], want, "sequence %d token %d" % (b, t)))
+
+
+@pytest.mark.parametrize("k_type", [O.TYPE_BF16, O.TYPE_F16])
+@pytest.mark.parametrize("n_head,groups", [(34, 2), (64, 2), (66, 2), (96, 2), (100, 4), (128, 4), (128, 2), (35, 1)])
+@pytest.mark.parametrize("paged", [False, True])
+def test_heads_of_a_short_decode_step_in_groups(gpu, k_type, n_head, groups, paged):
+    """More than 32 heads over few keys: groups of up to 32 (or 64) heads as sequences of their own on the same keys, Q with strides that
+    are not packed; ragged lengths with an empty sequence, the balanced page schedule and single pages; both passes of a 576-wide V."""
+    import torch
+    import jittorinfer_amd as J
+    rng = np.random.default_rng(n_head + groups)
+    if groups == 2 and n_head > 64:
+        lens = [2500, 900, 33, 1700] if paged else [2500] * 4      # too many tiles for groups of 32
+    else:
+        lens = [0, 129, 300, 31, 640, 1] if paged else [416] * 3
+    n_seq = len(lens)
+    if paged:
+        pool, bt, seqs = U.make_paged(rng, np.maximum(lens, 1), k_type)
+        seqs = [s[:l] for s, l in zip(seqs, lens)]
+        kw = dict(bt=bt, lens=lens)
+        pkw = dict(block_table=torch.from_numpy(bt).to(gpu), seq_lens=torch.tensor(lens, dtype=torch.int32, device=gpu))
+    else:
+        pool = U.encode_kv(rng.standard_normal((n_seq, lens[0], 576)).astype(np.float32), k_type)
+        seqs, kw, pkw = list(pool), {}, {}
+    q = rng.standard_normal((n_seq, n_head, 1, 576)).astype(np.float32)
+    info = J.plan(torch.from_numpy(q).to(gpu), torch.from_numpy(pool.view(np.int16)).to(gpu), k_type, dv=512, scale=U.SCALE, **pkw)
+    assert info["variant"] == 2 and (info["balanced"] == 1 or info["n_workgroups"] == groups * n_seq * info["n_splits"]), info
+    for dv in (512, 576):
+        got = _run(gpu, q, pool, k_type, dv=dv, scale=U.SCALE, **kw)[..., :dv]
+        for b in range(n_seq):
+            if len(seqs[b]) == 0:
+                assert np.isnan(got[b]).all()
+            else:
+                want = (O.flash_attn_ext_f64 if k_type == O.TYPE_F16 else O.flash_attn_ext)(q[b:b + 1], seqs[b][None], k_type, dv=dv, scale=U.SCALE)
+                print(dv, b, U.check(got[b:b + 1], want, "sequence %d" % b))
+    tq = torch.from_numpy(np.ascontiguousarray(q.transpose(1, 0, 2, 3))).to(gpu).permute(1, 0, 2, 3)   # [head][sequence] in memory
+    tp = torch.from_numpy(pool.view(np.int16)).to(gpu)
+    a = J.ggml_flash_attn_ext(tq, tp, k_type, dv=512, scale=U.SCALE, **pkw)[..., :512]
+    b = J.ggml_flash_attn_ext(torch.from_numpy(q).to(gpu), tp, k_type, dv=512, scale=U.SCALE, **pkw)[..., :512]
+    assert torch.equal(torch.nan_to_num(a), torch.nan_to_num(b))
