@@ -1,11 +1,14 @@
-"""Builds jittorinfer_amd/libggml-hip-mla.so (HIP kernels + C ABI + ggml backend plugin) for gfx950 with hipcc."""
+"""Builds jittorinfer_amd/libggml-hip-mla.so (HIP kernels + C ABI + ggml backend plugin) for gfx950 with hipcc, and
+jittorinfer_amd/_native.so (torch tensors -> C ABI, host code only) with g++."""
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libggml-hip-mla.so")
+NATIVE = os.path.join(HERE, "_native.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 COMMON = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
@@ -35,5 +38,15 @@ def build(verbose=False):
     return LIB
 
 
+def build_native():
+    import torch
+    from torch.utils import cpp_extension
+    torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI,
+          "-I" + sysconfig.get_paths()["include"]] + ["-isystem" + i for i in cpp_extension.include_paths()] +
+         [os.path.join(CSRC, "py_native.cpp"), "-o", NATIVE, "-L" + torch_lib, "-ltorch_python", "-ltorch_cpu", "-lc10"])
+    return NATIVE
+
+
 if __name__ == "__main__":
-    print(build(verbose="-v" in sys.argv))
+    print(build(verbose="-v" in sys.argv), build_native())

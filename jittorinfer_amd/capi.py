@@ -98,6 +98,27 @@ def library():
     return _lib
 
 
+_native = None
+
+
+def native():
+    """The module that takes torch tensors to the C ABI (csrc/py_native.cpp), bound to library(); raises if it has not been built."""
+    global _native
+    if _native is None:
+        import importlib
+        import torch
+        lib = library()
+        try:
+            mod = importlib.import_module("jittorinfer_amd._native")
+        except ImportError as e:
+            raise RuntimeError("jittorinfer_amd/_native.so is missing or does not load (%s): build it with `python jittorinfer_amd/build.py`" % e)
+        names = ("mla_attn_workspace_size", "mla_attn_launch", "mla_kv_write_launch", "mla_kv_write_rope_launch", "mla_rope_launch",
+                 "mla_mul_mat_launch", "mla_copy_f32_launch", "mla_front_batch_launch")
+        mod.bind(*[C.cast(getattr(lib, n), C.c_void_p).value for n in names], _workspace, _workspaces, torch._C._cuda_getCurrentRawStream)
+        _native = mod
+    return _native
+
+
 class MlaKvWriteArgs(C.Structure):
     """mla_kv_write_args of include/mla_kv_write.h."""
     _fields_ = [("n_tok", C.c_int32), ("src_type", C.c_int32), ("kv_type", C.c_int32), ("rows_type", C.c_int32),
@@ -199,15 +220,7 @@ def ggml_flash_attn_ext(q, k, kv_type, dv=512, mask=None, scale=1.0, max_bias=0.
     """GGML_OP_FLASH_ATTN_EXT of the reference (ggml_flash_attn_ext(ctx, q, k, v, mask, scale, max_bias,
     logit_softcap), ggml/src/ggml.c:3988) for the MLA shape, on the current torch stream.  v is the first `dv`
     columns of k's rows.  Returns dst in ggml's layout: float32 [n_seq, n_tok, n_head, 576] with dv columns valid."""
-    import torch
-    if not q.is_cuda:
-        raise RuntimeError("jittorinfer_amd runs on a gfx950 GPU only (there is no CPU path)")
-    a, out, keep = make_args(q, k, kv_type, dv, mask, scale, max_bias, logit_softcap, block_table, seq_lens, out, n_splits, flags, rows_per_wg, stream)
-    st = stream if stream is not None else torch.cuda.current_stream(q.device).cuda_stream
-    rc = library().mla_attn_launch(C.byref(a), C.c_void_p(st))
-    if rc != 0:
-        raise RuntimeError("mla_attn_launch failed with code %d" % rc)
-    return out
+    return (_native or native()).attn(q, k, kv_type, dv, mask, scale, max_bias, logit_softcap, block_table, seq_lens, out, n_splits, flags, rows_per_wg, stream)
 
 
 def plan(q, k, kv_type, **kw):
@@ -236,50 +249,10 @@ def kv_write(src, cache, kv_type, *, row0=None, rows=None, block_table=None, seq
     k_pe + rope: values 512 .. 575 of every row are k_pe (float32 [n_tok, 64], not yet rotated) rotated on the way
     (mla_kv_write_rope_launch); rope = dict(pos=..., and the keywords of ggml_rope_ext).  batch: a FrontBatch that takes
     the launch instead of the stream."""
-    import torch
-    if not src.is_cuda:
-        raise RuntimeError("jittorinfer_amd runs on a gfx950 GPU only (there is no CPU path)")
-    ra = None
-    if k_pe is not None:
-        ra = MlaKvWriteRopeArgs()
-        a = ra.w
-        kw = dict(rope)
-        rpos = kw.pop("pos")
-        assert k_pe.dtype == torch.float32 and k_pe.dim() == 2 and k_pe.shape == (src.shape[0], 64) and k_pe.stride(1) == 1
-        _fill_rope_args(ra.rope, k_pe.unsqueeze(1), rpos, k_pe.unsqueeze(1), **kw)
-    else:
-        a = MlaKvWriteArgs()
-    a.n_tok = src.shape[0]
-    a.kv_type = kv_type
-    a.src_type = MLA_TYPE_F32 if src.dtype == torch.float32 else kv_type
-    assert src.dim() == 2 and src.stride(1) == 1 and cache.dim() == 2 and cache.stride(1) == 1
-    assert cache.shape[1] * cache.element_size() == ROW_BYTES[kv_type]
-    if a.src_type == MLA_TYPE_F32:
-        assert src.shape[1] == 576 or (ra is not None and src.shape[1] >= 512)
-    else:
-        assert src.shape[1] * src.element_size() == ROW_BYTES[kv_type]
-    a.src, a.src_nb1 = src.data_ptr(), src.stride(0) * src.element_size()
-    a.kv, a.kv_nb1, a.n_kv_rows = cache.data_ptr(), cache.stride(0) * cache.element_size(), cache.shape[0]
-    assert (row0 is not None) + (rows is not None) + (block_table is not None) == 1
-    if row0 is not None:
-        a.row0 = row0
-    elif rows is not None:
-        assert rows.dtype in (torch.int32, torch.int64) and rows.is_contiguous() and rows.numel() == a.n_tok
-        a.rows, a.rows_type = rows.data_ptr(), 1 if rows.dtype == torch.int64 else 0
-    else:
-        for t in (block_table, seq_ids, positions):
-            assert t.dtype == torch.int32 and t.is_contiguous()
-        assert block_table.dim() == 2 and seq_ids.numel() == a.n_tok and positions.numel() == a.n_tok
-        a.block_table, a.bt_stride = block_table.data_ptr(), block_table.shape[1]
-        a.seq_ids, a.positions = seq_ids.data_ptr(), positions.data_ptr()
-    if batch is not None:
-        batch.add(MLA_FRONT_KV_WRITE_ROPE if ra is not None else MLA_FRONT_KV_WRITE, ra if ra is not None else a)
-        return cache
-    st = stream if stream is not None else torch.cuda.current_stream(src.device).cuda_stream
-    rc = library().mla_kv_write_rope_launch(C.byref(ra), C.c_void_p(st)) if ra is not None else library().mla_kv_write_launch(C.byref(a), C.c_void_p(st))
-    if rc != 0:
-        raise RuntimeError("mla_kv_write%s_launch failed with code %d" % ("_rope" if ra is not None else "", rc))
-    return cache
+    n = _native or native()
+    if k_pe is None:
+        return n.kv_write(src, cache, kv_type, row0, rows, block_table, seq_ids, positions, stream, batch, None)
+    return n.kv_write(src, cache, kv_type, row0, rows, block_table, seq_ids, positions, stream, batch, k_pe, *_rope_values(**rope))
 
 
 class MlaRopeArgs(C.Structure):
@@ -328,52 +301,17 @@ class FrontBatch:
         self.ops.append((kind, args))
 
     def launch(self, stream=None, device=None):
-        import torch
-        n = len(self.ops)
-        arr = (MlaFrontOp * max(n, 1))()
-        for i, (kind, args) in enumerate(self.ops):
-            arr[i].kind, arr[i].args = kind, C.addressof(args)
-        st = stream if stream is not None else torch.cuda.current_stream(device).cuda_stream
-        rc = library().mla_front_batch_launch(arr, n, C.c_void_p(st))
-        if rc != 0:
-            raise RuntimeError("mla_front_batch_launch failed with code %d" % rc)
+        n = _native or native()
+        if stream is None:
+            import torch
+            stream = torch.cuda.current_stream(device).cuda_stream if device is not None else torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+        n.front_batch(self.ops, stream)
         self.ops = []
 
 
-def _gpu_only(t):
-    if not t.is_cuda:
-        raise RuntimeError("jittorinfer_amd runs on a gfx950 GPU only (there is no CPU path)")
-
-
-def _stream(t, stream):
-    import torch
-    return stream if stream is not None else torch.cuda.current_stream(t.device).cuda_stream
-
-
-def _nb4(t):
-    """ggml-order byte strides / sizes of a torch tensor of up to 4 dims (last torch dim = ggml dim 0)."""
-    es = t.element_size()
-    ne = list(reversed(t.shape)) + [1] * (4 - t.dim())
-    nb = [s * es for s in reversed(t.stride())]
-    while len(nb) < 4:
-        nb.append(nb[-1] * ne[len(nb) - 1])
-    return ne, nb
-
-
-def _fill_rope_args(a, x, pos, out, *, n_dims, mode=0, n_ctx_orig=0, freq_base=10000.0, freq_scale=1.0, ext_factor=0.0, attn_factor=1.0,
-                    beta_fast=32.0, beta_slow=1.0, freq_factors=None):
-    import torch
-    assert pos.dtype == torch.int32 and pos.is_contiguous() and pos.numel() == x.shape[0]
-    ne, nb = _nb4(x)
-    _, dnb = _nb4(out)
-    a.src, a.dst, a.pos = x.data_ptr(), out.data_ptr(), pos.data_ptr()
-    a.ne[:], a.src_nb[:], a.dst_nb[:] = ne, nb, dnb
-    if freq_factors is not None:
-        assert freq_factors.dtype == torch.float32 and freq_factors.is_contiguous() and freq_factors.numel() >= n_dims // 2
-        a.freq_factors = freq_factors.data_ptr()
-    a.n_dims, a.mode, a.n_ctx_orig = n_dims, mode, n_ctx_orig
-    a.freq_base, a.freq_scale, a.ext_factor, a.attn_factor = freq_base, freq_scale, ext_factor, attn_factor
-    a.beta_fast, a.beta_slow = beta_fast, beta_slow
+def _rope_values(pos, n_dims, mode=0, n_ctx_orig=0, freq_base=10000.0, freq_scale=1.0, ext_factor=0.0, attn_factor=1.0,
+                 beta_fast=32.0, beta_slow=1.0, freq_factors=None):
+    return pos, n_dims, mode, n_ctx_orig, freq_base, freq_scale, ext_factor, attn_factor, beta_fast, beta_slow, freq_factors
 
 
 def ggml_rope_ext(x, pos, *, n_dims, mode=0, n_ctx_orig=0, freq_base=10000.0, freq_scale=1.0, ext_factor=0.0, attn_factor=1.0,
@@ -381,72 +319,21 @@ def ggml_rope_ext(x, pos, *, n_dims, mode=0, n_ctx_orig=0, freq_base=10000.0, fr
     """ggml_rope_ext (ggml/src/ggml.c:3495-3501) on the current torch stream.  x: float32 [n_tok, n_head, ne0] (ggml ne =
     {ne0, n_head, n_tok}), unit stride in the last dimension; pos: int32 [n_tok]; out: same shape (default: a new
     contiguous tensor; pass out=x to rotate in place)."""
-    import torch
-    _gpu_only(x)
-    assert x.dtype == torch.float32 and x.dim() == 3 and x.stride(2) == 1
-    assert pos.dtype == torch.int32 and pos.is_contiguous() and pos.numel() == x.shape[0]
-    if out is None:
-        out = torch.empty(x.shape, dtype=torch.float32, device=x.device)
-    assert out.shape == x.shape and out.dtype == torch.float32 and out.stride(2) == 1
-    a = MlaRopeArgs()
-    _fill_rope_args(a, x, pos, out, n_dims=n_dims, mode=mode, n_ctx_orig=n_ctx_orig, freq_base=freq_base, freq_scale=freq_scale,
-                    ext_factor=ext_factor, attn_factor=attn_factor, beta_fast=beta_fast, beta_slow=beta_slow, freq_factors=freq_factors)
-    if batch is not None:
-        batch.add(MLA_FRONT_ROPE, a)
-        return out
-    rc = library().mla_rope_launch(C.byref(a), C.c_void_p(_stream(x, stream)))
-    if rc != 0:
-        raise RuntimeError("mla_rope_launch failed with code %d" % rc)
-    return out
+    return (_native or native()).rope(x, out, stream, batch, pos, n_dims, mode, n_ctx_orig, freq_base, freq_scale, ext_factor, attn_factor,
+                                      beta_fast, beta_slow, freq_factors)
 
 
 def ggml_mul_mat(w, w_type, x, *, out=None, stream=None, batch=None):
     """ggml_mul_mat(src0 = w, src1 = x) for the absorb products (src/llama-graph-attn.cpp:264-275, :303-317).
     w: [w_ne2, N, K] 16-bit storage (bf16 / f16 bits, any 2-byte dtype), x: float32 [ne2, M, K], unit stride in the
     last dimension of both, ne2 % w_ne2 == 0; returns float32 [ne2, M, N]."""
-    import torch
-    _gpu_only(x)
-    assert w.dim() == 3 and x.dim() == 3 and w.element_size() == 2 and x.dtype == torch.float32
-    assert w.stride(2) == 1 and x.stride(2) == 1 and w.shape[2] == x.shape[2]
-    if out is None:
-        out = torch.empty((x.shape[0], x.shape[1], w.shape[1]), dtype=torch.float32, device=x.device)
-    assert out.shape == (x.shape[0], x.shape[1], w.shape[1]) and out.dtype == torch.float32 and out.stride(2) == 1
-    a = MlaMulMatArgs()
-    a.w_type, a.w, a.x, a.dst = w_type, w.data_ptr(), x.data_ptr(), out.data_ptr()
-    a.K, a.N, a.w_ne2, a.w_ne3 = w.shape[2], w.shape[1], w.shape[0], 1
-    a.M, a.ne2, a.ne3 = x.shape[1], x.shape[0], 1
-    a.w_nb1, a.w_nb2 = w.stride(1) * 2, w.stride(0) * 2
-    a.x_nb1, a.x_nb2 = x.stride(1) * 4, x.stride(0) * 4
-    a.d_nb1, a.d_nb2 = out.stride(1) * 4, out.stride(0) * 4
-    a.w_nb3, a.x_nb3, a.d_nb3 = a.w_nb2 * a.w_ne2, a.x_nb2 * a.ne2, a.d_nb2 * a.ne2
-    if batch is not None:
-        batch.add(MLA_FRONT_MUL_MAT, a)
-        return out
-    rc = library().mla_mul_mat_launch(C.byref(a), C.c_void_p(_stream(x, stream)))
-    if rc != 0:
-        raise RuntimeError("mla_mul_mat_launch failed with code %d" % rc)
-    return out
+    return (_native or native()).mul_mat(w, w_type, x, out, stream, batch)
 
 
 def copy_f32(src, dst, stream=None, batch=None):
     """Strided float32 copy (ggml_cont; each half of ggml_concat): dst[...] = src[...], same shape, any strides with a
     unit last one."""
-    import torch
-    _gpu_only(src)
-    assert src.dtype == torch.float32 and dst.dtype == torch.float32 and src.shape == dst.shape and src.dim() <= 4
-    assert src.stride(-1) == 1 and dst.stride(-1) == 1
-    a = MlaCopyArgs()
-    ne, nb = _nb4(src)
-    _, dnb = _nb4(dst)
-    a.src, a.dst = src.data_ptr(), dst.data_ptr()
-    a.ne[:], a.src_nb[:], a.dst_nb[:] = ne, nb, dnb
-    if batch is not None:
-        batch.add(MLA_FRONT_COPY, a)
-        return dst
-    rc = library().mla_copy_f32_launch(C.byref(a), C.c_void_p(_stream(src, stream)))
-    if rc != 0:
-        raise RuntimeError("mla_copy_f32_launch failed with code %d" % rc)
-    return dst
+    return (_native or native()).copy(src, dst, stream, batch)
 
 
 class PageTable:
