@@ -61,7 +61,8 @@ extern "C" {
                                       to f16 inside LDS and the f16 path runs (68 MFMAs): exact for values whose magnitude is
                                       0 or in [2^-14, 65504] (bf16 has fewer mantissa bits than f16), larger ones become
                                       +-65504, smaller ones lose bits below 2^-24; probabilities are rounded to f16.  Set it
-                                      for a cache that holds values outside that range. */
+                                      for a cache that holds values outside that range.  Without it, too, the tiles are multiplied
+                                      as they are where mask rows end before the block table's last page does. */
 
 /* errors */
 #define MLA_ERR_BAD_SHAPE     (-1)

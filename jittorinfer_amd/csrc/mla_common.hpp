@@ -147,6 +147,14 @@ inline int64_t key_capacity(const mla_attn_args * a) {
     return a->mask && a->mask_ne0 < n ? a->mask_ne0 : n;
 }
 
+// Mask rows that end before the block table's last page does (a block table has room for whole pages).
+inline bool narrow_mask(const mla_attn_args * a) { return a->mask && a->block_table && a->mask_ne0 < a->bt_stride * MLA_PAGE_TOKENS; }
+
+// bf16 cells on the programs that feed the probabilities as hi + lo halves and never convert a cell: asked for by flag, and under narrow
+// mask rows.  The general kernel took those launches, with the same halves; one f16 probability is 1.4e-4 off where they are 2e-6
+// off, and cells beyond f16's range would be cut.
+inline bool bf16_direct(const mla_attn_args * a) { return (a->flags & MLA_FLAG_BF16_DIRECT) || (a->kv_type == MLA_TYPE_BF16 && narrow_mask(a)); }
+
 // The pipelined decode kernel (mla_decode_kernel.hip); returns hipErrorInvalidValue for shapes it does not take.
 bool       decode_fast_applicable(const mla_attn_args * a);
 // Raises a kernel's dynamic-LDS limit to the 160 KB of a CU, once per device: the attribute belongs to the function on the

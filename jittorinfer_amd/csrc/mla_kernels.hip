@@ -475,15 +475,14 @@ __device__ __forceinline__ bool combine_row(const KParams & p, int & b, int & ro
 // flight together, and the weights of a group of splits are worked out once for both column groups.  A wave covers 16 rows x 4
 // column groups (twice): it reads runs of 256 bytes (16 rows of one column group are contiguous in the partial layout) and writes
 // 128 contiguous bytes per row.  grid = (ceil(rows/16), ceil(dv/256), n_seq), block = 256 = 16 rows x 16 column groups (x 2).
-template <bool TAIL>
 __global__ void __launch_bounds__(256) mla_attn_combine_kernel(const KParams p) {
-    int b = blockIdx.z, row = blockIdx.x * 16 + (threadIdx.x & 15);
+    const int b = blockIdx.z, row = blockIdx.x * 16 + (threadIdx.x & 15);
     const int cg  = blockIdx.y * 32 + (threadIdx.x >> 4);
-    if (!combine_row<TAIL>(p, b, row) || cg * 8 >= p.dv_total) return;
+    if (row >= p.n_rows || cg * 8 >= p.dv_total) return;
     const int seq_len = p.block_table ? min(p.seq_lens[b >> p.seq_shift], (int) p.bt_stride * MLA_PAGE_TOKENS) : (int) p.n_kv;
     const bool two = (cg + 16) * 8 < p.dv_total;   // the second column group exists
     int slot0, nvalid, lrow, slot_rows;
-    partial_slots<TAIL>(p, b, row, seq_len, slot0, nvalid, lrow, slot_rows);
+    partial_slots(p, b, row, seq_len, slot0, nvalid, lrow, slot_rows);
     if (nvalid < 0) return;
 
     const float2 *   ml = (const float2 *) p.part_ml + (int64_t) slot0 * slot_rows + lrow;
@@ -960,7 +959,7 @@ int validate(const mla_attn_args * a) {
 static bool token_form_candidate(const mla_attn_args * a, const Plan & pl) {
     if (a->n_head > 32 && a->kv_type != MLA_TYPE_Q8_0 && 128 % a->n_head == 0) return false;
     return pl.variant == 2 && pl.balanced == 2 && a->n_tok <= 256 && a->n_head <= 64 && (int64_t) a->n_tok * a->n_head > 32 && a->n_tok > 1 &&
-           pl.kvcopy_rows == 0 && !(a->flags & MLA_FLAG_BF16_DIRECT) && a->logit_softcap == 0.0f && !(a->max_bias > 0.0f);
+           pl.kvcopy_rows == 0 && !bf16_direct(a) && a->logit_softcap == 0.0f && !(a->max_bias > 0.0f);
 }
 static size_t token_image_bytes(const mla_attn_args * a) {
     return a->kv_type == MLA_TYPE_Q8_0 || a->n_head > 32 ? decode_fast_qpack_bytes(a->n_tok, 1) : 0;
@@ -970,17 +969,17 @@ static size_t token_image_bytes(const mla_attn_args * a) {
 // blocks of n_tiles 32-key tiles at most, in microseconds.  Fitted to launches measured on one box: a tile takes 1.33 us with few CUs
 // busy and 1.83 with all 256 (the chip's power limit), a workgroup 20 us beside its tiles (operands in, rows out, the scan of the
 // mask ahead), the pass that packs the operands of split row blocks and the merge of their partial rows 5 us + 0.1 per row block +
-// 0.01 per piece.  Measured: 8 row blocks x 94 tiles in 12 / 24 pieces each 40.7 / 35.2 us, 32 x 17 in 1 / 5 45.8 / 32.5, 108 x 32 in 2 / 3
+// `merge` per piece: 0.01, or 0.06 for the f32 partial rows of a tail (256 KB written and read again).  Measured: 8 row blocks x 94 tiles in 12 / 24 pieces each 40.7 / 35.2 us, 32 x 17 in 1 / 5 45.8 / 32.5, 108 x 32 in 2 / 3
 // 67.2 / 85.1 (3: a second round of workgroups), 108 x 103 in 2 / 3 126 / 162, 128 x 72 in 2 106, 26 x 129 in 9 59.4, 26 x 7 in 1 / 2 31.4 / 38.5.
-static double masked_split_cost(int64_t n_items, int64_t n_tiles, int64_t splits) {
+static double masked_split_cost(int64_t n_items, int64_t n_tiles, int64_t splits, double merge) {
     const int64_t pieces = n_items * splits, rounds = (pieces + 255) / 256;
     const double  busy = std::min(1.0, (double) pieces / 256), tile = 1.33 + 0.5 * busy;
-    return rounds * ((double) ((n_tiles + splits - 1) / splits) * tile + 20.0) + (splits > 1 ? 5.0 + 0.1 * n_items + 0.01 * pieces : 0.0);
+    return rounds * ((double) ((n_tiles + splits - 1) / splits) * tile + 20.0) + (splits > 1 ? 5.0 + 0.1 * n_items + merge * pieces : 0.0);
 }
-static int64_t masked_splits(int64_t n_items, int64_t n_tiles, int64_t most) {
+static int64_t masked_splits(int64_t n_items, int64_t n_tiles, int64_t most, double merge = 0.01) {
     int64_t best = 1;
     for (int64_t s = 2; s <= most && s <= n_tiles; s++)
-        if (masked_split_cost(n_items, n_tiles, s) < masked_split_cost(n_items, n_tiles, best)) best = s;
+        if (masked_split_cost(n_items, n_tiles, s, merge) < masked_split_cost(n_items, n_tiles, best, merge)) best = s;
     return best;
 }
 // One sequence in a contiguous cache, whose split form is the schedule that deals out equal runs of tiles: worth it from this many on.
@@ -1008,7 +1007,7 @@ int head_groups_shift(const mla_attn_args * a) {
 }
 
 // all_rows: of a sequence of the caller's (a may be the launch as the groups of heads make it)
-static int plan_rows(const mla_attn_args * a, Plan * pl, int64_t all_rows);
+static int plan_rows(const mla_attn_args * a, Plan * pl, int64_t all_rows, bool frugal);
 
 // The launch's own shape: the caller's, or with every group of heads a sequence.
 static mla_attn_args grouped(const mla_attn_args * a, int shift) {
@@ -1017,17 +1016,19 @@ static mla_attn_args grouped(const mla_attn_args * a, int shift) {
     return g;
 }
 
-int make_plan(const mla_attn_args * a, Plan * pl) {
+// frugal: for a caller whose scratch is fixed -- no partial rows that only save time (no groups of heads, no tail, no more splits of a
+// masked launch than give every CU a workgroup, narrow masks on the kernel that needs no operand image).
+int make_plan(const mla_attn_args * a, Plan * pl, bool frugal = false) {
     const int rc = validate(a);
     if (rc) return rc;
-    const int shift = head_groups_shift(a);
+    const int shift = frugal ? 0 : head_groups_shift(a);
     const mla_attn_args g = grouped(a, shift);
-    const int rc2 = plan_rows(&g, pl, (int64_t) a->n_tok * a->n_head);
+    const int rc2 = plan_rows(&g, pl, (int64_t) a->n_tok * a->n_head, frugal);
     pl->seq_shift = shift;
     return rc2;
 }
 
-static int plan_rows(const mla_attn_args * a, Plan * pl, int64_t all_rows) {
+static int plan_rows(const mla_attn_args * a, Plan * pl, int64_t all_rows, bool frugal) {
     const int64_t n_rows  = (int64_t) a->n_tok * a->n_head;
     int64_t max_len = a->block_table ? a->bt_stride * MLA_PAGE_TOKENS : a->n_kv;
     *pl = Plan{};
@@ -1045,7 +1046,7 @@ static int plan_rows(const mla_attn_args * a, Plan * pl, int64_t all_rows) {
         pl->split_tokens = (int) max_len;
         return 0;
     }
-    if (decode_fast_applicable(a) && a->rows_per_wg == 0) { max_len = key_capacity(a); pl->variant = 2; pl->n_passes = a->dv == 576 ? 2 : 1; pl->ndb = 16; pl->wm = 4; pl->wd = 1; }
+    if (decode_fast_applicable(a) && a->rows_per_wg == 0 && !(frugal && narrow_mask(a))) { max_len = key_capacity(a); pl->variant = 2; pl->n_passes = a->dv == 576 ? 2 : 1; pl->ndb = 16; pl->wm = 4; pl->wd = 1; }
     else if (a->dv == 576) { pl->n_passes = 2; pl->ndb = 9; pl->wm = 4; pl->wd = 1; }
     else {
         pl->n_passes = 1; pl->ndb = 16;
@@ -1065,17 +1066,18 @@ static int plan_rows(const mla_attn_args * a, Plan * pl, int64_t all_rows) {
         const int64_t wgs = (int64_t) a->n_seq * pl->n_row_blocks;
         splits = (256 + wgs - 1) / wgs;
         if (pl->wd > 1) splits *= 2;  // small-row shapes leave room for two workgroups per CU
-        if (pl->variant == 2 && a->mask) {
+        if (pl->variant == 2 && a->mask && !frugal) {
             const int64_t n_tiles = (max_len + TILE_TOK - 1) / TILE_TOK;
             if (n_rows <= 32)   splits = std::max<int64_t>(256 / wgs, 1);   // (the k-split program: short pieces, and no second round for the rest)
             else if (a->n_seq == 1 && !a->block_table) { if (!masked_worth_dealing(wgs, n_tiles)) splits = 1; }
             else if (wgs < 256) splits = masked_splits(wgs, n_tiles, 32);
             // More row blocks than whole rounds of 256 take: the ones left over would have the chip to themselves with most of it idle
             // (333 row blocks x 130 tiles: the 77 of the second round took nearly as long as the 256 of the first).  They are split, the
-            // others not: 449 -> 376 us; 300 x 50 tiles 172 -> 143 us, 280 x 259 848 -> 575 us, 400 x 138 464 -> 454 us.
-            if (wgs > 256 && wgs % 256 && !(a->flags & (MLA_FLAG_UNIFORM_SPLITS | MLA_FLAG_BF16_DIRECT)) && decode_fast_q8_copy_rows(a) == 0 &&
+            // others not: 463 -> 384 us; 300 x 50 tiles 188 -> 166 us, 280 x 259 849 -> 580 us, 217 x 31 139 -> 73 us (f32 partial rows: an output row
+            // that was never rounded to 16 bits in between still is not).
+            if (wgs > 256 && wgs % 256 && !(a->flags & MLA_FLAG_UNIFORM_SPLITS) && !bf16_direct(a) && decode_fast_q8_copy_rows(a) == 0 &&
                 a->logit_softcap == 0.0f && !(a->max_bias > 0.0f)) {   // (what the tail builds of the kernel take)
-                const int64_t n_tail = wgs % 256, best = masked_splits(n_tail, n_tiles, 8);
+                const int64_t n_tail = wgs % 256, best = masked_splits(n_tail, n_tiles, 8, 0.06);
                 if (best > 1) { pl->tail_first = (int) (wgs - n_tail); pl->tail_splits = (int) best; }
             }
         }
@@ -1157,7 +1159,8 @@ static int plan_rows(const mla_attn_args * a, Plan * pl, int64_t all_rows) {
         const size_t n_slots = pl->tail_splits ? n_tail * pl->tail_splits : pl->balanced ? (size_t) pl->n_wg + pl->n_units : (size_t) a->n_seq * pl->n_splits;
         const size_t slot_rows = pl->balanced == 2 || pl->tail_splits ? 128 : (size_t) n_rows;
         const size_t n_part = n_slots * slot_rows * (pl->variant == 2 ? 512 : a->dv);
-        pl->part_f32   = n_part * sizeof(float) <= ((size_t) 32 << 20);
+        // (a tail's rows would be whole without it, with no partial at all: theirs are f32 at any size)
+        pl->part_f32   = pl->tail_splits || n_part * sizeof(float) <= ((size_t) 32 << 20);
         pl->ws_part_o  = n_part * (pl->part_f32 ? sizeof(float) : sizeof(_Float16));
         pl->ws_part_ml = n_slots * slot_rows * 2 * sizeof(float);
     }
@@ -1220,9 +1223,9 @@ int mla_attn_plan(const mla_attn_args * args, mla_attn_plan_info * out) {
 
 // phases: bit 0 = the attention kernels (partials or final output), bit 1 = the combine pass,
 // bit 2 = the small passes ahead of the pipelined kernel (Q operand image, key extent of the mask)
-static int launch_phases(const mla_attn_args * args, void * stream, int phases) {
+static int launch_phases(const mla_attn_args * args, void * stream, int phases, bool frugal = false) {
     Plan pl;
-    const int rc = make_plan(args, &pl);
+    const int rc = make_plan(args, &pl, frugal);
     if (rc) return rc;
     const mla_attn_args launch = grouped(args, pl.seq_shift), * a = &launch;
     const size_t need = plan_ws(pl);
@@ -1252,7 +1255,7 @@ static int launch_phases(const mla_attn_args * args, void * stream, int phases) 
     kp.part_f32 = pl.part_f32;
     kp.rel_splits = a->mask != nullptr && (pl.variant == 2 || pl.ws_maskext > 0);
     kp.balanced = pl.balanced; kp.n_wg = pl.n_wg; kp.n_seq_sched = a->n_seq; kp.n_units = pl.n_units;
-    kp.bf16_direct = (a->flags & MLA_FLAG_BF16_DIRECT) ? 1 : 0;
+    kp.bf16_direct = bf16_direct(a) ? 1 : 0;
     kp.slot_rows = pl.balanced == 2 || pl.tail_splits ? 128 : kp.n_rows;
     kp.tail_first = pl.tail_first; kp.tail_splits = pl.tail_splits;
     kp.part_ml = (float *) (ws + align256(pl.ws_part_o));
@@ -1333,9 +1336,8 @@ static int launch_phases(const mla_attn_args * args, void * stream, int phases) 
             hipLaunchKernelGGL(mla_attn_combine_wide_kernel<4>, gw, dim3(256), 0, st, kp);
             return (int) hipGetLastError();
         }
-        dim3 g((c_rows + 15) / 16, (unsigned) ((dv + 255) / 256), c_seq);
-        auto kern = pl.tail_splits ? mla_attn_combine_kernel<true> : mla_attn_combine_kernel<false>;
-        hipLaunchKernelGGL(kern, g, dim3(256), 0, st, kp);
+        dim3 g((unsigned) ((kp.n_rows + 15) / 16), (unsigned) ((dv + 255) / 256), (unsigned) a->n_seq);
+        hipLaunchKernelGGL(mla_attn_combine_kernel, g, dim3(256), 0, st, kp);
         return (int) hipGetLastError();
     };
     if (pl.variant == 2) {
@@ -1397,12 +1399,14 @@ int mla_attn_launch_static(const mla_attn_args * a, void * stream) {
     b.workspace      = nullptr;
     b.workspace_size = 0;
     Plan pl;
-    const int rc = make_plan(&b, &pl);
+    int rc = make_plan(&b, &pl);
+    const bool frugal = !rc && plan_ws(pl) > MLA_ATTN_STATIC_WORKSPACE_MAX;
+    if (frugal) rc = make_plan(&b, &pl, true);
     if (rc) return rc;
     if (plan_ws(pl) > MLA_ATTN_STATIC_WORKSPACE_MAX) return MLA_ERR_TOO_LARGE;
     b.workspace      = ptr;
     b.workspace_size = MLA_ATTN_STATIC_WORKSPACE_MAX;
-    return launch_phases(&b, stream, 7);
+    return launch_phases(&b, stream, 7, frugal);
 }
 int mla_attn_launch_partials(const mla_attn_args * a, void * stream) { return launch_phases(a, stream, 5); }
 int mla_attn_launch_kernel(const mla_attn_args * a, void * stream) { return launch_phases(a, stream, 1); }

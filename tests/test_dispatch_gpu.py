@@ -57,7 +57,7 @@ def test_row_blocks_left_over_from_whole_rounds_are_split(gpu, k_type, n_seq, n_
     rng = np.random.default_rng(n_new + n_seq)
     lens = [n_old + n_new - 40 * b for b in range(n_seq)]
     q8s = 1.0 / 32 if k_type == O.TYPE_Q8_0 else None
-    width = (max(lens) + 31) // 32 * 32
+    width = (max(lens) + 127) // 128 * 128 if n_seq > 1 else (max(lens) + 31) // 32 * 32
     q = rng.standard_normal((n_seq, n_head, n_new, 576)).astype(np.float32)
     if n_seq > 1:
         pool, bt, seqs = U.make_paged(rng, lens, k_type, q8_scale=q8s)
@@ -124,3 +124,51 @@ def test_heads_of_a_short_decode_step_in_groups(gpu, k_type, n_head, groups, pag
     a = J.ggml_flash_attn_ext(tq, tp, k_type, dv=512, scale=U.SCALE, **pkw)[..., :512]
     b = J.ggml_flash_attn_ext(torch.from_numpy(q).to(gpu), tp, k_type, dv=512, scale=U.SCALE, **pkw)[..., :512]
     assert torch.equal(torch.nan_to_num(a), torch.nan_to_num(b))
+
+
+def test_narrow_mask_rows_of_bf16_cells_keep_both_halves_of_the_probabilities(gpu):
+    """Probabilities as hi + lo bf16 halves carry 16 bits (errors of 2^-18 on average), one f16 probability 11 (2^-13, 1.4e-4 in relative L2
+    over a row): 3e-5 lies between.  And cells beyond the range of f16 are multiplied as they are."""
+    rng = np.random.default_rng(3)
+    n_head, n_new, width = 16, 9, 160
+    lens = [n_new + 150, n_new + 149]
+    for big in (False, True):
+        pool, bt, seqs = U.make_paged(rng, lens, O.TYPE_BF16)
+        q = rng.standard_normal((2, n_head, n_new, 576)).astype(np.float32)
+        if big:   # value columns 500 .. 511 of every cell at 2^20 and above; Q is 0 there
+            for x in (pool, *seqs):
+                x[..., 500:512] = (x[..., 500:512] & 0x807f) | 0x4980
+            q[..., 500:512] = 0
+        mask = _causal_mask(n_new, max(lens), width)
+        got = _run(gpu, q, pool, O.TYPE_BF16, mask=mask, bt=bt, lens=lens, scale=U.SCALE)[..., :512]
+        want = _want(q, [s[:width] for s in seqs], O.TYPE_BF16, mask)
+        print(U.check(got, want, "narrow mask rows", max_abs=2.0 ** 21 if big else 2e-4, rel_l2=3e-5))
+
+
+@pytest.mark.parametrize("n_seq,n_new,width,paged", [(1, 290, 640, False), (2, 288, 31968, True)])
+def test_static_scratch_takes_what_fits_without_the_rows_that_only_save_time(gpu, n_seq, n_new, width, paged):
+    """290 row blocks whose tail's partial rows do not fit the fixed scratch beside the operand image, and 2 x 36 behind narrow mask rows whose
+    seven splits do not: both run, as the launch that needs neither."""
+    import ctypes as C
+    import torch
+    import jittorinfer_amd as J
+    lib = J.library()
+    rng = np.random.default_rng(n_new)
+    n_head = 16 if paged else 128
+    lens = [width - 3] * n_seq
+    q = torch.from_numpy(rng.standard_normal((n_seq, n_head, n_new, 576)).astype(np.float32)).to(gpu)
+    if paged:
+        pool, bt, _ = U.make_paged(rng, lens, O.TYPE_F16)
+        kw = dict(block_table=torch.from_numpy(bt).to(gpu), seq_lens=torch.tensor(lens, dtype=torch.int32, device=gpu))
+    else:
+        pool, kw = U.encode_kv(rng.standard_normal((1, width, 576)).astype(np.float32), O.TYPE_F16), {}
+    k = torch.from_numpy(pool.view(np.int16)).to(gpu)
+    mask = torch.from_numpy(_causal_mask(n_new, width - 3, width).view(np.float16)).to(gpu)
+    out = torch.full((n_seq, n_new, n_head, 512), float("nan"), dtype=torch.float32, device=gpu)
+    a, _, keep = J.capi.make_args(q, k, J.MLA_TYPE_F16, dv=512, scale=U.SCALE, mask=mask, out=out, **kw)
+    assert lib.mla_attn_workspace_size(C.byref(a)) > J.capi.MLA_ATTN_STATIC_WORKSPACE_MAX
+    a.workspace, a.workspace_size = None, 0
+    assert lib.mla_attn_launch_static(C.byref(a), C.c_void_p(torch.cuda.current_stream(gpu).cuda_stream)) == 0
+    want = J.ggml_flash_attn_ext(q, k, J.MLA_TYPE_F16, dv=512, scale=U.SCALE, mask=mask, flags=J.MLA_FLAG_UNIFORM_SPLITS, **kw)
+    torch.cuda.synchronize()
+    print(U.check(out.cpu().numpy(), want.cpu().numpy()[..., :512], "fixed scratch"))
