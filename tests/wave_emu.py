@@ -819,6 +819,17 @@ def _(w, o, m):
     w.wv(o[0], r.astype(U32))
 
 
+@op("v_lshl_add_u64")
+def _(w, o, m):
+    def u64(x):
+        if x[0] == "v":
+            return w.rv(x).astype(np.uint64) | w.rv(x, 1).astype(np.uint64) << np.uint64(32)
+        return np.full(64, w.rs(x, 2), np.uint64)
+    r = (u64(o[1]) << np.uint64(w.rs(o[2]))) + u64(o[3])
+    w.wv(o[0], r.astype(U32))
+    w.wv(o[0], (r >> np.uint64(32)).astype(U32), 1)
+
+
 @op("v_addc_co_u32")
 def _(w, o, m):
     r = w.rv(o[2]).astype(np.uint64) + w.rv(o[3]).astype(np.uint64) + _bits(w.rs(o[4], 2)).astype(np.uint64)
