@@ -1110,10 +1110,12 @@ bool decode_fast_applicable(const mla_attn_args * a) {
     if (a->kv_type != MLA_TYPE_Q8_0 && a->kv_nb1 != ROW_BYTES) return false;   // (the f16 copy of a Q8_0 cache is packed by construction)
     if (a->mask) {
         // whole tiles only (no key past n_kv is touched in a mask row), 32-bit offsets into the mask, 8-byte aligned loads
-        // A mask row may be narrower than the cache -- a prompt chunk of several sequences brings rows as wide as the longest of them, its
-        // block table has room for whole pages: keys past the row's end count as masked, so the row's end is the cache's
+        // Over pages a mask row may be narrower than the table has room for -- a prompt chunk of several sequences brings rows as wide as
+        // the longest of them: keys past the row's end count as masked, so the row's end is the cache's
         // (2 sequences x 537 new tokens x 64 heads, rows of 544 over pages of 640: 1023 us on the general kernel, 180 here).
+        // Over a contiguous cache the caller sets the number of rows: a mask narrower than that stays on the general kernel.
         const int64_t n_kv = key_capacity(a);
+        if (!a->block_table && a->mask_ne0 < a->n_kv) return false;
         if (n_kv % TILE_TOK || (a->mask_nb1 & 7) || ((uintptr_t) a->mask & 7)) return false;
         if ((int64_t) a->n_tok * a->mask_nb1 >= (1ll << 31)) return false;
     }

@@ -172,3 +172,20 @@ def test_static_scratch_takes_what_fits_without_the_rows_that_only_save_time(gpu
     want = J.ggml_flash_attn_ext(q, k, J.MLA_TYPE_F16, dv=512, scale=U.SCALE, mask=mask, flags=J.MLA_FLAG_UNIFORM_SPLITS, **kw)
     torch.cuda.synchronize()
     print(U.check(out.cpu().numpy(), want.cpu().numpy()[..., :512], "fixed scratch"))
+
+
+@pytest.mark.parametrize("big", [False, True])
+@pytest.mark.parametrize("n_seq", [1, 2])
+def test_narrow_mask_rows_over_a_contiguous_cache_keep_both_halves_too(gpu, n_seq, big):
+    """The same bound for a cache without a block table (640 cells, mask rows of 544), with cells inside and beyond f16's range."""
+    rng = np.random.default_rng(n_seq)
+    n_head, n_new, n_kv, width = 16, 9, 640, 544
+    k = U.encode_kv(rng.standard_normal((n_seq, n_kv, 576)).astype(np.float32), O.TYPE_BF16)
+    q = rng.standard_normal((n_seq, n_head, n_new, 576)).astype(np.float32)
+    if big:
+        k[..., 500:512] = (k[..., 500:512] & 0x807f) | 0x4980
+        q[..., 500:512] = 0
+    mask = _causal_mask(n_new, width - 7, width)
+    got = _run(gpu, q, k, O.TYPE_BF16, mask=mask, scale=U.SCALE)[..., :512]
+    want = _want(q, [s[:width] for s in k], O.TYPE_BF16, mask)
+    print(U.check(got, want, "narrow mask rows, contiguous", max_abs=2.0 ** 21 if big else 2e-4, rel_l2=3e-5))

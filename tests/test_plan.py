@@ -1,0 +1,48 @@
+"""What the planner of the attention launches decides, on the CPU: pointers are made up, nothing is launched."""
+import ctypes as C
+
+import pytest
+
+import jittorinfer_amd.capi as J
+
+BF16, F16, Q8_0 = J.MLA_TYPE_BF16, J.MLA_TYPE_F16, J.MLA_TYPE_Q8_0
+
+
+def _args(n_seq, n_tok, n_head, keys, kv_type=BF16, paged=True, mask_width=0, dv=512, flags=0, n_splits=0):
+    """The argument block of a launch over `keys` cells per sequence; mask_width 0: no mask."""
+    a = J.MlaAttnArgs()
+    a.n_seq, a.n_head, a.n_tok, a.dk, a.dv = n_seq, n_head, n_tok, 576, dv
+    a.q_type, a.kv_type, a.flags, a.scale, a.n_splits = J.MLA_TYPE_F32, kv_type, flags, 0.07, n_splits
+    a.q, a.kv, a.dst = 1 << 20, 1 << 30, 1 << 31
+    a.q_nb2, a.q_nb1, a.q_nb3 = 2304, 2304 * n_head, 2304 * n_head * n_tok
+    a.kv_nb1, a.dst_nb1 = J.ROW_BYTES[kv_type], dv * 4
+    if paged:
+        a.bt_stride = (keys + 127) // 128
+        a.n_kv, a.block_table, a.seq_lens = n_seq * a.bt_stride * 128, 1 << 20, 1 << 20
+    else:
+        a.n_kv, a.kv_nb3 = keys, a.kv_nb1 * keys if n_seq > 1 else 0
+    if mask_width:
+        a.mask, a.mask_nb1, a.mask_ne0 = 1 << 20, mask_width * 2, mask_width
+    return a
+
+
+def _plan(*args, **kw):
+    info = J.MlaPlanInfo()
+    a = _args(*args, **kw)
+    assert J.library().mla_attn_plan(C.byref(a), C.byref(info)) == 0
+    return info
+
+
+def _workspace(*args, **kw):
+    a = _args(*args, **kw)
+    return J.library().mla_attn_workspace_size(C.byref(a))
+
+
+@pytest.mark.parametrize("kv_type", [BF16, F16, Q8_0])
+@pytest.mark.parametrize("n_seq,n_tok,n_head", [(1, 9, 16), (2, 9, 16), (1, 64, 128), (3, 2, 16)])
+def test_a_mask_narrower_than_a_contiguous_cache_is_the_general_kernel_s(kv_type, n_seq, n_tok, n_head):
+    """It multiplies the cells as they are, with both halves of the probabilities, and keeps small partials in f32."""
+    assert _plan(n_seq, n_tok, n_head, 4096, kv_type, paged=False, mask_width=2048).variant == 0
+    assert _plan(n_seq, n_tok, n_head, 4096, kv_type, paged=False, mask_width=4096).variant == 2
+    assert _plan(n_seq, n_tok, n_head, 4096, kv_type, paged=False, mask_width=8192).variant == 2
+    assert _workspace(n_seq, n_tok, n_head, 4096, kv_type, paged=False, mask_width=2048) <= J.MLA_ATTN_STATIC_WORKSPACE_MAX
