@@ -1006,8 +1006,8 @@ int head_groups_shift(const mla_attn_args * a) {
     return a->n_head > 64 && a->n_head % 2 == 0 && a->n_seq <= 128 && tiles <= 2048 && tiles * a->n_seq <= 16000 ? 1 : 0;
 }
 
-// all_rows: of a sequence of the caller's (a may be the launch as the groups of heads make it)
-static int plan_rows(const mla_attn_args * a, Plan * pl, int64_t all_rows, bool frugal);
+// all_rows: of a sequence of the caller's (a may be the launch as the groups of heads make it); pipelined: not only the general kernel
+static int plan_rows(const mla_attn_args * a, Plan * pl, int64_t all_rows, bool frugal, bool pipelined);
 
 // The launch's own shape: the caller's, or with every group of heads a sequence.
 static mla_attn_args grouped(const mla_attn_args * a, int shift) {
@@ -1023,12 +1023,20 @@ int make_plan(const mla_attn_args * a, Plan * pl, bool frugal = false) {
     if (rc) return rc;
     const int shift = frugal ? 0 : head_groups_shift(a);
     const mla_attn_args g = grouped(a, shift);
-    const int rc2 = plan_rows(&g, pl, (int64_t) a->n_tok * a->n_head, frugal);
+    const int64_t all_rows = (int64_t) a->n_tok * a->n_head;
+    const bool narrow = narrow_mask(a);
+    const int rc2 = plan_rows(&g, pl, all_rows, frugal, !(frugal && narrow));
     pl->seq_shift = shift;
+    // Narrow mask rows whose splits would leave f16 partial rows on the pipelined kernel (more pages than a split can list, or more
+    // splits) and whole rows or f32 partials on the general one, which these launches came from, stay there.
+    if (!rc2 && narrow && pl->variant == 2 && pl->n_splits > 1 && !pl->part_f32) {
+        Plan general;
+        if (!plan_rows(&g, &general, all_rows, frugal, false) && (general.n_splits == 1 || general.part_f32)) *pl = general;
+    }
     return rc2;
 }
 
-static int plan_rows(const mla_attn_args * a, Plan * pl, int64_t all_rows, bool frugal) {
+static int plan_rows(const mla_attn_args * a, Plan * pl, int64_t all_rows, bool frugal, bool pipelined) {
     const int64_t n_rows  = (int64_t) a->n_tok * a->n_head;
     int64_t max_len = a->block_table ? a->bt_stride * MLA_PAGE_TOKENS : a->n_kv;
     *pl = Plan{};
@@ -1046,7 +1054,7 @@ static int plan_rows(const mla_attn_args * a, Plan * pl, int64_t all_rows, bool 
         pl->split_tokens = (int) max_len;
         return 0;
     }
-    if (decode_fast_applicable(a) && a->rows_per_wg == 0 && !(frugal && narrow_mask(a))) { max_len = key_capacity(a); pl->variant = 2; pl->n_passes = a->dv == 576 ? 2 : 1; pl->ndb = 16; pl->wm = 4; pl->wd = 1; }
+    if (pipelined && decode_fast_applicable(a) && a->rows_per_wg == 0) { max_len = key_capacity(a); pl->variant = 2; pl->n_passes = a->dv == 576 ? 2 : 1; pl->ndb = 16; pl->wm = 4; pl->wd = 1; }
     else if (a->dv == 576) { pl->n_passes = 2; pl->ndb = 9; pl->wm = 4; pl->wd = 1; }
     else {
         pl->n_passes = 1; pl->ndb = 16;

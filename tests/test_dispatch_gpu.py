@@ -189,3 +189,22 @@ def test_narrow_mask_rows_over_a_contiguous_cache_keep_both_halves_too(gpu, n_se
     got = _run(gpu, q, k, O.TYPE_BF16, mask=mask, scale=U.SCALE)[..., :512]
     want = _want(q, [s[:width] for s in k], O.TYPE_BF16, mask)
     print(U.check(got, want, "narrow mask rows, contiguous", max_abs=2.0 ** 21 if big else 2e-4, rel_l2=3e-5))
+
+
+@pytest.mark.parametrize("n_seq,n_new,n_head,dv,n_pages", [(256, 1, 128, 576, 66), (278, 1, 24, 512, 128)])
+def test_narrow_mask_rows_over_many_pages_keep_f32_rows(gpu, n_seq, n_new, n_head, dv, n_pages):
+    """More pages than a split of the pipelined kernel can list: its splits would leave f16 partial rows (2^-12 of each, 1e-4 over a
+    row) where the general kernel has whole rows or f32 partials.  One pool of pages that all the sequences share; bf16 cells and
+    probabilities as hi + lo halves: 3e-5 as above."""
+    rng = np.random.default_rng(n_head + dv)
+    width = n_pages * 128 - 32
+    lens = [int(x) for x in rng.integers(width - 200, width, n_seq)]
+    k = U.encode_kv(rng.standard_normal((n_pages * 128, 576)).astype(np.float32), O.TYPE_BF16)
+    bt = np.stack([rng.permutation(n_pages) for _ in range(n_seq)]).astype(np.int32)
+    q = rng.standard_normal((n_seq, n_head, n_new, 576)).astype(np.float32)
+    mask = _causal_mask(n_new, width, width)
+    got = _run(gpu, q, k, O.TYPE_BF16, dv=dv, mask=mask, bt=bt, lens=lens, scale=U.SCALE)[..., :dv]
+    for b in (0, n_seq // 2, n_seq - 1):
+        cells = np.concatenate([k[p * 128:(p + 1) * 128] for p in bt[b]])[:lens[b]]
+        want = O.flash_attn_ext(q[b:b + 1], cells[None], O.TYPE_BF16, dv=dv, mask=np.ascontiguousarray(mask[:, :lens[b]]), scale=U.SCALE)
+        print(U.check(got[b:b + 1], want, "sequence %d" % b, rel_l2=3e-5))

@@ -46,3 +46,11 @@ def test_a_mask_narrower_than_a_contiguous_cache_is_the_general_kernel_s(kv_type
     assert _plan(n_seq, n_tok, n_head, 4096, kv_type, paged=False, mask_width=4096).variant == 2
     assert _plan(n_seq, n_tok, n_head, 4096, kv_type, paged=False, mask_width=8192).variant == 2
     assert _workspace(n_seq, n_tok, n_head, 4096, kv_type, paged=False, mask_width=2048) <= J.MLA_ATTN_STATIC_WORKSPACE_MAX
+
+
+@pytest.mark.parametrize("kv_type", [BF16, F16])
+@pytest.mark.parametrize("n_seq,n_tok,n_head,dv,n_pages", [(256, 1, 128, 576, 66), (4, 1661, 48, 576, 265), (278, 1, 24, 512, 128)])
+def test_narrow_masks_over_many_pages_gain_no_f16_partial_rows(kv_type, n_seq, n_tok, n_head, dv, n_pages):
+    """Where the general kernel has whole rows or f32 partials.  With fewer pages the pipelined kernel has too, and takes them."""
+    assert _plan(n_seq, n_tok, n_head, n_pages * 128, kv_type, mask_width=n_pages * 128 - 32, dv=dv).variant == 0
+    assert _plan(n_seq, n_tok, n_head, 20 * 128, kv_type, mask_width=20 * 128 - 32, dv=dv).variant == 2
