@@ -155,6 +155,16 @@ inline bool narrow_mask(const mla_attn_args * a) { return a->mask && a->block_ta
 // off, and cells beyond f16's range would be cut.
 inline bool bf16_direct(const mla_attn_args * a) { return (a->flags & MLA_FLAG_BF16_DIRECT) || (a->kv_type == MLA_TYPE_BF16 && narrow_mask(a)); }
 
+// 16-bit cells: rows per sequence whose launches run on the column-split programs (decode_cs_applicable has the reasons).
+inline bool decode_cs_rows(int64_t n_rows) {
+    const int64_t tail = n_rows % 128;
+    return tail == 0 || tail > 96 || n_rows > 128;
+}
+
+// What the builds with a tail of shared row blocks (KParams::tail_splits) take of a masked launch on the pipelined kernel: raw Q8_0 tiles, or
+// 16-bit cells on the column-split programs; no bias.  The planner gives no other launch a tail, the launcher refuses one.
+bool decode_has_tail_build(const mla_attn_args * a);
+
 // The pipelined decode kernel (mla_decode_kernel.hip); returns hipErrorInvalidValue for shapes it does not take.
 bool       decode_fast_applicable(const mla_attn_args * a);
 // Raises a kernel's dynamic-LDS limit to the 160 KB of a CU, once per device: the attribute belongs to the function on the

@@ -1125,6 +1125,11 @@ bool decode_fast_applicable(const mla_attn_args * a) {
     return true;
 }
 
+bool decode_has_tail_build(const mla_attn_args * a) {
+    if (!a->mask || a->logit_softcap != 0.0f || a->max_bias > 0.0f || bf16_direct(a)) return false;
+    return a->kv_type == MLA_TYPE_Q8_0 ? decode_fast_q8_copy_rows(a) == 0 : decode_cs_rows((int64_t) a->n_tok * a->n_head);
+}
+
 // Q8_0 rows -> f16 rows: value = f16(q * f32(d)), one rounding of an exact product, the operand the Q8_0 wave program
 // builds in LDS.  One thread = 8 values (a quarter of a block): grid = ceil(rows * 72 / 256).
 __global__ void __launch_bounds__(NTHREADS) mla_q8_to_f16_kernel(const char * src, int64_t src_nb1, int64_t src_nb3, int64_t rows_per_batch,
@@ -1175,8 +1180,7 @@ constexpr int64_t STREAM_CACHE_BYTES = 96ll << 20;   // (three times what the ei
 static bool decode_cs_applicable(const KParams & kp, int kv_type) {
     if (kv_type != MLA_TYPE_BF16 && kv_type != MLA_TYPE_F16) return false;
     if (kp.bf16_direct || kp.q_as_q8) return false;
-    const int tail = kp.n_rows % 128;
-    return (tail == 0 || tail > 96 || kp.n_rows > 128) && kp.slot_rows < (1 << 22);
+    return decode_cs_rows(kp.n_rows) && kp.slot_rows < (1 << 22);
 }
 
 // 33 .. 64 rows per sequence (a decode step of a model with 48 or 64 heads per device), no mask: the column-split program for two row
@@ -1299,7 +1303,7 @@ hipError_t launch_decode_fast(const KParams & kp_in, int kv_type, dim3 grid, hip
         if (cs) return kv_type == MLA_TYPE_F16 ? launch_variant<SRC_F16_CSB, true>(kp, grid, st) : launch_variant<SRC_BF16_CSB, true>(kp, grid, st);
         return kv_type == MLA_TYPE_F16 ? launch_variant<SRC_F16, true, false, true>(kp, grid, st) : launch_variant<SRC_BF16_CVT, true, false, true>(kp, grid, st);
     }
-    if (kp.tail_splits) {   // (make_plan gives the others no tail)
+    if (kp.tail_splits) {   // (decode_has_tail_build: the planner gives the others no tail)
         if (!m || bias || kp.q_as_q8 || kp.balanced || kp.n_splits != 1) return hipErrorInvalidValue;
         if (kv_type == MLA_TYPE_Q8_0) return launch_variant<SRC_Q8, true, false, false, true>(kp, grid, st);
         if (!cs || !q_in_kernel) return hipErrorInvalidValue;

@@ -1083,8 +1083,7 @@ static int plan_rows(const mla_attn_args * a, Plan * pl, int64_t all_rows, bool 
             // (333 row blocks x 130 tiles: the 77 of the second round took nearly as long as the 256 of the first).  They are split, the
             // others not: 463 -> 384 us; 300 x 50 tiles 188 -> 166 us, 280 x 259 849 -> 580 us, 217 x 31 139 -> 73 us (f32 partial rows: an output row
             // that was never rounded to 16 bits in between still is not).
-            if (wgs > 256 && wgs % 256 && !(a->flags & MLA_FLAG_UNIFORM_SPLITS) && !bf16_direct(a) && decode_fast_q8_copy_rows(a) == 0 &&
-                a->logit_softcap == 0.0f && !(a->max_bias > 0.0f)) {   // (what the tail builds of the kernel take)
+            if (wgs > 256 && wgs % 256 && !(a->flags & MLA_FLAG_UNIFORM_SPLITS) && decode_has_tail_build(a)) {
                 const int64_t n_tail = wgs % 256, best = masked_splits(n_tail, n_tiles, 8, 0.06);
                 if (best > 1) { pl->tail_first = (int) (wgs - n_tail); pl->tail_splits = (int) best; }
             }

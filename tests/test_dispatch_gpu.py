@@ -208,3 +208,27 @@ def test_narrow_mask_rows_over_many_pages_keep_f32_rows(gpu, n_seq, n_new, n_hea
         cells = np.concatenate([k[p * 128:(p + 1) * 128] for p in bt[b]])[:lens[b]]
         want = O.flash_attn_ext(q[b:b + 1], cells[None], O.TYPE_BF16, dv=dv, mask=np.ascontiguousarray(mask[:, :lens[b]]), scale=U.SCALE)
         print(U.check(got[b:b + 1], want, "sequence %d" % b, rel_l2=3e-5))
+
+
+@pytest.mark.parametrize("k_type", [O.TYPE_BF16, O.TYPE_F16, O.TYPE_Q8_0])
+@pytest.mark.parametrize("n_seq,n_head,n_new,paged", [(300, 16, 1, True), (288, 16, 4, False), (300, 64, 1, True), (300, 96, 1, False), (300, 97, 1, True), (260, 48, 3, True)])
+def test_more_masked_sequences_than_workgroups(gpu, k_type, n_seq, n_head, n_new, paged):
+    """More than 256 masked sequences of 16 to 144 rows: those beyond whole rounds of workgroups are split where the program of their
+    rows has a build for it (Q8_0 cells, more than 96 rows), and have a workgroup each where it does not."""
+    rng = np.random.default_rng(n_seq + n_head)
+    n_kv = 768
+    q8s = 1.0 / 32 if k_type == O.TYPE_Q8_0 else None
+    q = rng.standard_normal((n_seq, n_head, n_new, 576)).astype(np.float32)
+    mask = _causal_mask(n_new, n_kv, n_kv)
+    if paged:   # one pool of pages that all the sequences share
+        k = U.encode_kv(rng.standard_normal((9 * 128, 576)).astype(np.float32), k_type, q8_scale=q8s)
+        bt = np.stack([rng.permutation(9)[:n_kv // 128] for _ in range(n_seq)]).astype(np.int32)
+        lens = [n_kv - b % 100 for b in range(n_seq)]
+        cells = lambda b: np.concatenate([k[p * 128:(p + 1) * 128] for p in bt[b]])[:lens[b]]
+        kw = dict(bt=bt, lens=lens)
+    else:
+        k = U.encode_kv(rng.standard_normal((n_seq, n_kv, 576)).astype(np.float32), k_type, q8_scale=q8s)
+        cells, kw = (lambda b: k[b]), {}
+    got = _run(gpu, q, k, k_type, mask=mask, scale=U.SCALE, **kw)[..., :512]
+    for b in (0, 255, 256, n_seq - 1):
+        print(b, U.check(got[b:b + 1], _want(q[b:b + 1], [cells(b)], k_type, mask), "sequence %d" % b))

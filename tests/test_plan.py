@@ -54,3 +54,13 @@ def test_narrow_masks_over_many_pages_gain_no_f16_partial_rows(kv_type, n_seq, n
     """Where the general kernel has whole rows or f32 partials.  With fewer pages the pipelined kernel has too, and takes them."""
     assert _plan(n_seq, n_tok, n_head, n_pages * 128, kv_type, mask_width=n_pages * 128 - 32, dv=dv).variant == 0
     assert _plan(n_seq, n_tok, n_head, 20 * 128, kv_type, mask_width=20 * 128 - 32, dv=dv).variant == 2
+
+
+@pytest.mark.parametrize("kv_type", [BF16, F16, Q8_0])
+@pytest.mark.parametrize("paged", [False, True])
+@pytest.mark.parametrize("n_tok,n_head", [(1, 16), (2, 16), (4, 16), (1, 64), (1, 96), (3, 1), (1, 97), (1, 128), (1, 130), (3, 48)])
+def test_a_tail_only_where_the_kernel_has_a_build_for_it(kv_type, paged, n_tok, n_head):
+    """300 masked sequences: 44 row blocks (or 88 of the two-block ones) beyond whole rounds of 256.  Column-split programs and Q8_0 tiles."""
+    n_blocks = 300 * ((n_tok * n_head + 127) // 128)
+    has_build = kv_type == Q8_0 or n_tok * n_head > 96
+    assert (_plan(300, n_tok, n_head, 2048, kv_type, paged=paged, mask_width=2048).n_workgroups > n_blocks) == has_build
