@@ -2,6 +2,8 @@
 // tensors, fills the argument block and launches.  Filling a ctypes structure field by field took 6 us of a 13 us attention call and
 // most of the 70 us a layer of a decode step spent on the host, more than its kernels run for small batches; here it takes
 // under 1 us a call.  Every function takes its arguments by position; capi.py gives them names and defaults.
+// What torch throws (out of memory, a tensor without strides or storage) ends at entry<>, as the Python exception torch itself would
+// raise; every reference and buffer taken on the way has an owner that gives it back.
 #include <Python.h>
 
 #include <string.h>
@@ -10,7 +12,9 @@
 #include <vector>
 
 #include <ATen/ops/empty.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/utils/object_ptr.h>
 
 #include "../../include/mla_attn.h"
 #include "../../include/mla_front.h"
@@ -21,11 +25,13 @@ namespace {
 constexpr int PAGE = MLA_PAGE_TOKENS;
 
 // A launch may wait for room in the device's queue: other Python threads run meanwhile.
-template <typename F> int unlocked(F f) {
+struct Unlocked {
     PyThreadState * t = PyEval_SaveThread();
-    const int rc = f();
-    PyEval_RestoreThread(t);
-    return rc;
+    ~Unlocked() { PyEval_RestoreThread(t); }
+};
+template <typename F> int unlocked(F f) {
+    const Unlocked u;
+    return f();
 }
 
 // The library's entry points, the Python layer's workspace table and what grows it, torch's raw current stream: handed over by bind().
@@ -81,13 +87,10 @@ bool stream_of(PyObject * o, const at::Tensor & t, void *& st) {
         st = PyLong_AsVoidPtr(o);
         return !PyErr_Occurred();
     }
-    PyObject * idx = PyLong_FromLong(t.device().index());
-    if (!idx) return false;
-    PyObject * raw = PyObject_CallOneArg(lib.raw_stream, idx);
-    Py_DECREF(idx);
+    THPObjectPtr idx(PyLong_FromLong(t.device().index()));
+    THPObjectPtr raw(idx ? PyObject_CallOneArg(lib.raw_stream, idx.get()) : nullptr);
     if (!raw) return false;
-    st = PyLong_AsVoidPtr(raw);
-    Py_DECREF(raw);
+    st = PyLong_AsVoidPtr(raw.get());
     return !PyErr_Occurred();
 }
 // ggml-order sizes and byte strides of a tensor of up to 4 dimensions (last torch dimension = ggml dimension 0)
@@ -99,30 +102,24 @@ void nb4(const at::Tensor & t, int64_t ne[4], int64_t nb[4]) {
 }
 int64_t row_bytes(long kv_type) { return kv_type == MLA_TYPE_F16 || kv_type == MLA_TYPE_BF16 ? 1152 : kv_type == MLA_TYPE_Q8_0 ? 612 : -1; }
 
-// The scratch area of (device, stream): a look-up in the Python layer's table; too small or missing, the Python layer makes one.
-bool workspace(PyObject * q, void * st, size_t need, mla_attn_args & a) {
-    PyObject * dev = PyObject_GetAttrString(q, "device");
-    if (!dev) return false;
-    PyObject * handle = PyLong_FromVoidPtr(st), * key = handle ? PyTuple_Pack(2, dev, handle) : nullptr, * ws = nullptr;
-    bool ok = key != nullptr;
-    if (ok) {
-        ws = PyDict_GetItemWithError(lib.workspaces, key);
-        ok = !PyErr_Occurred();
-        Py_XINCREF(ws);
+// The scratch area of (device, stream): a look-up in the Python layer's table; too small or missing, the Python layer makes one.  The
+// caller keeps what is returned until its launch is queued: another thread may give areas back meanwhile.
+THPObjectPtr workspace(PyObject * q, void * st, size_t need, mla_attn_args & a) {
+    THPObjectPtr dev(PyObject_GetAttrString(q, "device")), handle(dev ? PyLong_FromVoidPtr(st) : nullptr);
+    THPObjectPtr key(handle ? PyTuple_Pack(2, dev.get(), handle.get()) : nullptr);
+    if (!key) return THPObjectPtr();
+    PyObject * const found = PyDict_GetItemWithError(lib.workspaces, key.get());
+    if (!found && PyErr_Occurred()) return THPObjectPtr();
+    THPObjectPtr ws(Py_XNewRef(found));
+    if (!ws || (size_t) THPVariable_Unpack(ws.get()).numel() < need) {
+        THPObjectPtr n(PyLong_FromSize_t(need));
+        ws = n ? PyObject_CallFunctionObjArgs(lib.workspace, dev.get(), n.get(), handle.get(), nullptr) : nullptr;
+        if (!ws) return ws;
     }
-    if (ok && (!ws || (size_t) THPVariable_Unpack(ws).numel() < need)) {
-        Py_XDECREF(ws);
-        PyObject * n = PyLong_FromSize_t(need);
-        ws = n ? PyObject_CallFunctionObjArgs(lib.workspace, dev, n, handle, nullptr) : nullptr;
-        Py_XDECREF(n);
-        ok = ws && THPVariable_Check(ws);
-    }
-    if (ok) {
-        const at::Tensor & t = THPVariable_Unpack(ws);
-        a.workspace = t.data_ptr(); a.workspace_size = (size_t) t.numel();
-    }
-    Py_XDECREF(ws); Py_XDECREF(key); Py_XDECREF(handle); Py_DECREF(dev);
-    return ok;
+    const at::Tensor * t = tensor(ws.get());
+    if (!t) return THPObjectPtr();
+    a.workspace = t->data_ptr(); a.workspace_size = (size_t) t->numel();
+    return ws;
 }
 
 // attn(q, k, kv_type, dv, mask, scale, max_bias, logit_softcap, block_table, seq_lens, out, n_splits, flags, rows_per_wg, stream) -> out
@@ -169,7 +166,9 @@ PyObject * attn(PyObject *, PyObject * const * v, Py_ssize_t n) {
     REQUIRE(out.scalar_type() == at::kFloat && out.dim() == 4 && out.is_contiguous() && out.size(0) == n_seq && out.size(1) == n_tok && out.size(2) == n_head && out.size(3) >= a.dv);
     a.dst = (float *) out.data_ptr(); a.dst_nb1 = out.size(3) * 4;
     void * st;
-    if (!stream_of(v[14], q, st) || !workspace(v[0], st, lib.workspace_size(&a), a)) return nullptr;
+    if (!stream_of(v[14], q, st)) return nullptr;
+    THPObjectPtr ws = workspace(v[0], st, lib.workspace_size(&a), a);
+    if (!ws) return nullptr;
     const int rc = unlocked([&] { return lib.attn(&a, st); });
     if (rc) return failed("mla_attn_launch", rc);
     if (made.defined()) return THPVariable_Wrap(made);
@@ -179,13 +178,10 @@ PyObject * attn(PyObject *, PyObject * const * v, Py_ssize_t n) {
 
 // The argument block of an op of a batch: kept as bytes by the batch until it is launched.
 PyObject * add_to_batch(PyObject * batch, int kind, const void * args, size_t size, PyObject * result) {
-    PyObject * k = PyLong_FromLong(kind), * b = PyBytes_FromStringAndSize((const char *) args, (Py_ssize_t) size), * name = PyUnicode_InternFromString("add"), * r = nullptr;
-    if (k && b && name) r = PyObject_CallMethodObjArgs(batch, name, k, b, nullptr);
-    Py_XDECREF(k); Py_XDECREF(b); Py_XDECREF(name);
-    if (!r) return nullptr;
-    Py_DECREF(r);
-    Py_INCREF(result);
-    return result;
+    THPObjectPtr k(PyLong_FromLong(kind)), b(PyBytes_FromStringAndSize((const char *) args, (Py_ssize_t) size)), name(PyUnicode_InternFromString("add"));
+    if (!k || !b || !name) return nullptr;
+    THPObjectPtr r(PyObject_CallMethodObjArgs(batch, name.get(), k.get(), b.get(), nullptr));
+    return r ? Py_NewRef(result) : nullptr;
 }
 
 // values: pos, n_dims, mode, n_ctx_orig, freq_base, freq_scale, ext_factor, attn_factor, beta_fast, beta_slow, freq_factors
@@ -224,18 +220,14 @@ PyObject * rope(PyObject *, PyObject * const * v, Py_ssize_t n) {
     mla_rope_args a;
     memset(&a, 0, sizeof a);
     if (!fill_rope(a, x, out, v + 4, x.size(0))) return nullptr;
-    PyObject * result = made.defined() ? THPVariable_Wrap(made) : Py_NewRef(v[1]);
+    THPObjectPtr result(made.defined() ? THPVariable_Wrap(made) : Py_NewRef(v[1]));
     if (!result) return nullptr;
-    if (v[3] != Py_None) {
-        PyObject * r = add_to_batch(v[3], MLA_FRONT_ROPE, &a, sizeof a, result);
-        Py_DECREF(result);
-        return r;
-    }
+    if (v[3] != Py_None) return add_to_batch(v[3], MLA_FRONT_ROPE, &a, sizeof a, result.get());
     void * st;
-    if (!stream_of(v[2], x, st)) { Py_DECREF(result); return nullptr; }
+    if (!stream_of(v[2], x, st)) return nullptr;
     const int rc = unlocked([&] { return lib.rope(&a, st); });
-    if (rc) { Py_DECREF(result); return failed("mla_rope_launch", rc); }
-    return result;
+    if (rc) return failed("mla_rope_launch", rc);
+    return result.release();
 }
 
 // mul_mat(w, w_type, x, out, stream, batch) -> out
@@ -261,18 +253,14 @@ PyObject * mul_mat(PyObject *, PyObject * const * v, Py_ssize_t n) {
     a.w_nb1 = w.stride(1) * 2; a.w_nb2 = w.stride(0) * 2; a.w_nb3 = a.w_nb2 * a.w_ne2;
     a.x_nb1 = x.stride(1) * 4; a.x_nb2 = x.stride(0) * 4; a.x_nb3 = a.x_nb2 * a.ne2;
     a.d_nb1 = out.stride(1) * 4; a.d_nb2 = out.stride(0) * 4; a.d_nb3 = a.d_nb2 * a.ne2;
-    PyObject * result = made.defined() ? THPVariable_Wrap(made) : Py_NewRef(v[3]);
+    THPObjectPtr result(made.defined() ? THPVariable_Wrap(made) : Py_NewRef(v[3]));
     if (!result) return nullptr;
-    if (v[5] != Py_None) {
-        PyObject * r = add_to_batch(v[5], MLA_FRONT_MUL_MAT, &a, sizeof a, result);
-        Py_DECREF(result);
-        return r;
-    }
+    if (v[5] != Py_None) return add_to_batch(v[5], MLA_FRONT_MUL_MAT, &a, sizeof a, result.get());
     void * st;
-    if (!stream_of(v[4], x, st)) { Py_DECREF(result); return nullptr; }
+    if (!stream_of(v[4], x, st)) return nullptr;
     const int rc = unlocked([&] { return lib.mul_mat(&a, st); });
-    if (rc) { Py_DECREF(result); return failed("mla_mul_mat_launch", rc); }
-    return result;
+    if (rc) return failed("mla_mul_mat_launch", rc);
+    return result.release();
 }
 
 // copy(src, dst, stream, batch) -> dst
@@ -353,32 +341,34 @@ PyObject * kv_write(PyObject *, PyObject * const * v, Py_ssize_t n) {
     return Py_NewRef(v[1]);
 }
 
+struct Buffers {
+    std::vector<Py_buffer> held;
+    ~Buffers() { for (Py_buffer & b : held) PyBuffer_Release(&b); }
+};
+
 // front_batch(ops, stream): ops = [(kind, argument block: bytes or anything with a buffer), ...]
 PyObject * front_batch(PyObject *, PyObject * const * v, Py_ssize_t n) {
     if (!arg_count(n, 2)) return nullptr;
     REQUIRE(PyList_Check(v[0]));
     const Py_ssize_t count = PyList_GET_SIZE(v[0]);
     std::vector<mla_front_op> ops((size_t) std::max<Py_ssize_t>(count, 1));
-    std::vector<Py_buffer>    held;
-    held.reserve((size_t) count);
-    bool ok = true;
-    for (Py_ssize_t i = 0; i < count && ok; i++) {
+    Buffers b;
+    b.held.reserve((size_t) count);
+    for (Py_ssize_t i = 0; i < count; i++) {
         PyObject * op = PyList_GET_ITEM(v[0], i);
         Py_buffer  buf;
-        ok = PyTuple_Check(op) && PyTuple_GET_SIZE(op) == 2 && PyObject_GetBuffer(PyTuple_GET_ITEM(op, 1), &buf, PyBUF_SIMPLE) == 0;
-        if (!ok) break;
-        held.push_back(buf);
+        if (!PyTuple_Check(op) || PyTuple_GET_SIZE(op) != 2) {
+            PyErr_SetString(PyExc_TypeError, "front_batch: ops are (kind, argument block) pairs");
+            return nullptr;
+        }
+        if (PyObject_GetBuffer(PyTuple_GET_ITEM(op, 1), &buf, PyBUF_SIMPLE) != 0) return nullptr;
+        b.held.push_back(buf);
         ops[(size_t) i] = mla_front_op{ (int32_t) PyLong_AsLong(PyTuple_GET_ITEM(op, 0)), 0, buf.buf };
-        ok = !PyErr_Occurred();
+        if (PyErr_Occurred()) return nullptr;
     }
-    void * st = ok ? PyLong_AsVoidPtr(v[1]) : nullptr;
-    ok = ok && !PyErr_Occurred();
-    const int rc = ok ? unlocked([&] { return lib.front_batch(ops.data(), (int32_t) count, st); }) : 0;
-    for (Py_buffer & b : held) PyBuffer_Release(&b);
-    if (!ok) {
-        if (!PyErr_Occurred()) PyErr_SetString(PyExc_TypeError, "front_batch: ops are (kind, argument block) pairs");
-        return nullptr;
-    }
+    void * st = PyLong_AsVoidPtr(v[1]);
+    if (PyErr_Occurred()) return nullptr;
+    const int rc = unlocked([&] { return lib.front_batch(ops.data(), (int32_t) count, st); });
     if (rc) return failed("mla_front_batch_launch", rc);
     Py_RETURN_NONE;
 }
@@ -398,7 +388,13 @@ PyObject * bind(PyObject *, PyObject * const * v, Py_ssize_t n) {
     Py_RETURN_NONE;
 }
 
-#define FAST(name) { #name, (PyCFunction) (void (*)(void)) name, METH_FASTCALL, nullptr }
+template <PyObject * (*F)(PyObject *, PyObject * const *, Py_ssize_t)> PyObject * entry(PyObject * self, PyObject * const * v, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    return F(self, v, n);
+    END_HANDLE_TH_ERRORS
+}
+
+#define FAST(name) { #name, (PyCFunction) (void (*)(void)) entry<name>, METH_FASTCALL, nullptr }
 PyMethodDef methods[] = { FAST(bind), FAST(attn), FAST(rope), FAST(mul_mat), FAST(copy), FAST(kv_write), FAST(front_batch), { nullptr, nullptr, 0, nullptr } };
 PyModuleDef module = { PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr };
 
