@@ -1084,7 +1084,9 @@ static int plan_rows(const mla_attn_args * a, Plan * pl, int64_t all_rows, bool 
             // others not: 463 -> 384 us; 300 x 50 tiles 188 -> 166 us, 280 x 259 849 -> 580 us, 217 x 31 139 -> 73 us (f32 partial rows: an output row
             // that was never rounded to 16 bits in between still is not).
             if (wgs > 256 && wgs % 256 && !(a->flags & MLA_FLAG_UNIFORM_SPLITS) && decode_has_tail_build(a)) {
-                const int64_t n_tail = wgs % 256, best = masked_splits(n_tail, n_tiles, 8, 0.06);
+                // At most 512 pieces of 256 KB: 128 MB of partial rows, whatever the launch (200 blocks in 7 pieces each would
+                // leave 350 MB for a tenth of one round).
+                const int64_t n_tail = wgs % 256, best = masked_splits(n_tail, n_tiles, std::min<int64_t>(8, 512 / n_tail), 0.06);
                 if (best > 1) { pl->tail_first = (int) (wgs - n_tail); pl->tail_splits = (int) best; }
             }
         }

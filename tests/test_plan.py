@@ -64,3 +64,12 @@ def test_a_tail_only_where_the_kernel_has_a_build_for_it(kv_type, paged, n_tok, 
     n_blocks = 300 * ((n_tok * n_head + 127) // 128)
     has_build = kv_type == Q8_0 or n_tok * n_head > 96
     assert (_plan(300, n_tok, n_head, 2048, kv_type, paged=paged, mask_width=2048).n_workgroups > n_blocks) == has_build
+
+
+@pytest.mark.parametrize("kv_type", [BF16, F16, Q8_0])
+@pytest.mark.parametrize("n_tok", [257, 300, 356, 384, 464, 470, 480, 490, 511, 1000])
+def test_a_tail_s_partial_rows_are_bounded(kv_type, n_tok):
+    """A prompt chunk of n_tok row blocks behind 65536 cells: the tail adds at most 128 MB (and (m, l) pairs) to what the launch takes without."""
+    kw = dict(paged=False, mask_width=65536)
+    more = _workspace(1, n_tok, 128, 65536, kv_type, **kw) - _workspace(1, n_tok, 128, 65536, kv_type, flags=J.MLA_FLAG_UNIFORM_SPLITS, **kw)
+    assert 0 <= more <= (128 << 20) + 512 * 128 * 8 + 512
