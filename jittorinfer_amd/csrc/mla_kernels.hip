@@ -1082,8 +1082,10 @@ static int plan_rows(const mla_attn_args * a, Plan * pl, int64_t all_rows, bool 
             // More row blocks than whole rounds of 256 take: the ones left over would have the chip to themselves with most of it idle
             // (333 row blocks x 130 tiles: the 77 of the second round took nearly as long as the 256 of the first).  They are split, the
             // others not: 463 -> 384 us; 300 x 50 tiles 188 -> 166 us, 280 x 259 849 -> 580 us, 217 x 31 139 -> 73 us (f32 partial rows: an output row
-            // that was never rounded to 16 bits in between still is not).
-            if (wgs > 256 && wgs % 256 && !(a->flags & MLA_FLAG_UNIFORM_SPLITS) && decode_has_tail_build(a)) {
+            // that was never rounded to 16 bits in between still is not).  Below 12 rounds: beyond, the one left over is too small a part of the
+            // launch for the merge (without / with a tail: 3948 row blocks x 80 tiles 1789 / 1840 us, 3393 x 36 1064 / 1081, 5644 x 48 2232 / 2230,
+            // but 2874 x 96 2589 / 2516).
+            if (wgs > 256 && wgs < 12 * 256 && wgs % 256 && !(a->flags & MLA_FLAG_UNIFORM_SPLITS) && decode_has_tail_build(a)) {
                 // At most 512 pieces of 256 KB: 128 MB of partial rows, whatever the launch (200 blocks in 7 pieces each would
                 // leave 350 MB for a tenth of one round).
                 const int64_t n_tail = wgs % 256, best = masked_splits(n_tail, n_tiles, std::min<int64_t>(8, 512 / n_tail), 0.06);

@@ -73,3 +73,8 @@ def test_a_tail_s_partial_rows_are_bounded(kv_type, n_tok):
     kw = dict(paged=False, mask_width=65536)
     more = _workspace(1, n_tok, 128, 65536, kv_type, **kw) - _workspace(1, n_tok, 128, 65536, kv_type, flags=J.MLA_FLAG_UNIFORM_SPLITS, **kw)
     assert 0 <= more <= (128 << 20) + 512 * 128 * 8 + 512
+
+
+def test_a_launch_of_many_rounds_has_no_tail():
+    for n_tok, tail in ((256 + 40, True), (11 * 256 + 40, True), (12 * 256 + 40, False), (20 * 256 + 40, False)):
+        assert (_plan(1, n_tok, 128, 8192, F16, paged=False, mask_width=8192).n_workgroups > n_tok) == tail
