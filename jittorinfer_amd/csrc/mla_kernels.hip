@@ -1036,6 +1036,8 @@ int make_plan(const mla_attn_args * a, Plan * pl, bool frugal = false) {
     return rc2;
 }
 
+constexpr int64_t PART_F32_MAX = 32 << 20;   // f32 partials up to here, f16 beyond
+
 static int plan_rows(const mla_attn_args * a, Plan * pl, int64_t all_rows, bool frugal, bool pipelined) {
     const int64_t n_rows  = (int64_t) a->n_tok * a->n_head;
     int64_t max_len = a->block_table ? a->bt_stride * MLA_PAGE_TOKENS : a->n_kv;
@@ -1078,7 +1080,12 @@ static int plan_rows(const mla_attn_args * a, Plan * pl, int64_t all_rows, bool 
             const int64_t n_tiles = (max_len + TILE_TOK - 1) / TILE_TOK;
             if (n_rows <= 32)   splits = std::max<int64_t>(256 / wgs, 1);   // (the k-split program: short pieces, and no second round for the rest)
             else if (a->n_seq == 1 && !a->block_table) { if (!masked_worth_dealing(wgs, n_tiles)) splits = 1; }
-            else if (wgs < 256) splits = masked_splits(wgs, n_tiles, 32);
+            else if (wgs < 256) {
+                // (partials that are f32 with a workgroup for every CU stay f32: no more splits than that allows)
+                const int64_t split_bytes = (int64_t) a->n_seq * n_rows * 512 * sizeof(float), fill_pages = (n_pages + splits - 1) / splits;
+                const bool f32 = (n_pages + fill_pages - 1) / fill_pages * split_bytes <= PART_F32_MAX;
+                splits = masked_splits(wgs, n_tiles, f32 ? std::min<int64_t>(32, PART_F32_MAX / split_bytes) : 32);
+            }
             // More row blocks than whole rounds of 256 take: the ones left over would have the chip to themselves with most of it idle
             // (333 row blocks x 130 tiles: the 77 of the second round took nearly as long as the 256 of the first).  They are split, the
             // others not: 463 -> 384 us; 300 x 50 tiles 188 -> 166 us, 280 x 259 849 -> 580 us, 217 x 31 139 -> 73 us (f32 partial rows: an output row
@@ -1171,7 +1178,7 @@ static int plan_rows(const mla_attn_args * a, Plan * pl, int64_t all_rows, bool 
         const size_t slot_rows = pl->balanced == 2 || pl->tail_splits ? 128 : (size_t) n_rows;
         const size_t n_part = n_slots * slot_rows * (pl->variant == 2 ? 512 : a->dv);
         // (a tail's rows would be whole without it, with no partial at all: theirs are f32 at any size)
-        pl->part_f32   = pl->tail_splits || n_part * sizeof(float) <= ((size_t) 32 << 20);
+        pl->part_f32   = pl->tail_splits || n_part * sizeof(float) <= (size_t) PART_F32_MAX;
         pl->ws_part_o  = n_part * (pl->part_f32 ? sizeof(float) : sizeof(_Float16));
         pl->ws_part_ml = n_slots * slot_rows * 2 * sizeof(float);
     }

@@ -78,3 +78,11 @@ def test_a_tail_s_partial_rows_are_bounded(kv_type, n_tok):
 def test_a_launch_of_many_rounds_has_no_tail():
     for n_tok, tail in ((256 + 40, True), (11 * 256 + 40, True), (12 * 256 + 40, False), (20 * 256 + 40, False)):
         assert (_plan(1, n_tok, 128, 8192, F16, paged=False, mask_width=8192).n_workgroups > n_tok) == tail
+
+
+@pytest.mark.parametrize("n_seq,n_tok,n_head,keys,paged", [(73, 2, 24, 24352, False), (157, 3, 16, 11904, True), (66, 1, 48, 18176, True), (2, 17, 16, 16896, False)])
+def test_more_splits_of_a_masked_launch_keep_f32_partials(n_seq, n_tok, n_head, keys, paged):
+    """Where as many splits as give every CU a workgroup have f32 partials, the splits taken instead have too."""
+    kw = dict(paged=paged, mask_width=keys)
+    splits, rows = _plan(n_seq, n_tok, n_head, keys, F16, **kw).n_splits, n_tok * n_head
+    assert splits > 1 and _workspace(n_seq, n_tok, n_head, keys, F16, **kw) >= n_seq * splits * rows * 512 * 4
