@@ -969,16 +969,16 @@ static size_t token_image_bytes(const mla_attn_args * a) {
 // blocks of n_tiles 32-key tiles at most, in microseconds.  Fitted to launches measured on one box: a tile takes 1.33 us with few CUs
 // busy and 1.83 with all 256 (the chip's power limit), a workgroup 20 us beside its tiles (operands in, rows out, the scan of the
 // mask ahead), the pass that packs the operands of split row blocks and the merge of their partial rows 5 us + 0.1 per row block +
-// `merge` per piece: 0.01, or 0.06 for the f32 partial rows of a tail (256 KB written and read again).  Measured: 8 row blocks x 94 tiles in 12 / 24 pieces each 40.7 / 35.2 us, 32 x 17 in 1 / 5 45.8 / 32.5, 108 x 32 in 2 / 3
+// `merge` per piece: 0.01, 0.06 for the f32 partial rows of a tail (256 KB written and read again), 0.08 for 128 f32 rows of few row blocks.  Measured: 8 row blocks x 94 tiles in 12 / 24 pieces each 40.7 / 35.2 us, 32 x 17 in 1 / 5 45.8 / 32.5, 108 x 32 in 2 / 3
 // 67.2 / 85.1 (3: a second round of workgroups), 108 x 103 in 2 / 3 126 / 162, 128 x 72 in 2 106, 26 x 129 in 9 59.4, 26 x 7 in 1 / 2 31.4 / 38.5.
 static double masked_split_cost(int64_t n_items, int64_t n_tiles, int64_t splits, double merge) {
     const int64_t pieces = n_items * splits, rounds = (pieces + 255) / 256;
     const double  busy = std::min(1.0, (double) pieces / 256), tile = 1.33 + 0.5 * busy;
     return rounds * ((double) ((n_tiles + splits - 1) / splits) * tile + 20.0) + (splits > 1 ? 5.0 + 0.1 * n_items + merge * pieces : 0.0);
 }
-static int64_t masked_splits(int64_t n_items, int64_t n_tiles, int64_t most, double merge = 0.01) {
-    int64_t best = 1;
-    for (int64_t s = 2; s <= most && s <= n_tiles; s++)
+static int64_t masked_splits(int64_t n_items, int64_t n_tiles, int64_t most, double merge = 0.01, int64_t least = 1) {
+    int64_t best = least;
+    for (int64_t s = least + 1; s <= most && s <= n_tiles; s++)
         if (masked_split_cost(n_items, n_tiles, s, merge) < masked_split_cost(n_items, n_tiles, best, merge)) best = s;
     return best;
 }
@@ -1007,7 +1007,7 @@ int head_groups_shift(const mla_attn_args * a) {
 }
 
 // all_rows: of a sequence of the caller's (a may be the launch as the groups of heads make it); pipelined: not only the general kernel
-static int plan_rows(const mla_attn_args * a, Plan * pl, int64_t all_rows, bool frugal, bool pipelined);
+static int plan_rows(const mla_attn_args * a, Plan * pl, int64_t all_rows, int frugal, bool pipelined);
 
 // The launch's own shape: the caller's, or with every group of heads a sequence.
 static mla_attn_args grouped(const mla_attn_args * a, int shift) {
@@ -1016,9 +1016,9 @@ static mla_attn_args grouped(const mla_attn_args * a, int shift) {
     return g;
 }
 
-// frugal: for a caller whose scratch is fixed -- no partial rows that only save time (no groups of heads, no tail, no more splits of a
-// masked launch than give every CU a workgroup, narrow masks on the kernel that needs no operand image).
-int make_plan(const mla_attn_args * a, Plan * pl, bool frugal = false) {
+// frugal: for a caller whose scratch is fixed -- no partial rows that only save time (no groups of heads, no tail, as many splits of a
+// masked launch as give every CU a workgroup, or with 2 as few of those as pay; narrow masks on the kernel that needs no operand image).
+int make_plan(const mla_attn_args * a, Plan * pl, int frugal = 0) {
     const int rc = validate(a);
     if (rc) return rc;
     const int shift = frugal ? 0 : head_groups_shift(a);
@@ -1038,7 +1038,7 @@ int make_plan(const mla_attn_args * a, Plan * pl, bool frugal = false) {
 
 constexpr int64_t PART_F32_MAX = 32 << 20;   // f32 partials up to here, f16 beyond
 
-static int plan_rows(const mla_attn_args * a, Plan * pl, int64_t all_rows, bool frugal, bool pipelined) {
+static int plan_rows(const mla_attn_args * a, Plan * pl, int64_t all_rows, int frugal, bool pipelined) {
     const int64_t n_rows  = (int64_t) a->n_tok * a->n_head;
     int64_t max_len = a->block_table ? a->bt_stride * MLA_PAGE_TOKENS : a->n_kv;
     *pl = Plan{};
@@ -1071,20 +1071,32 @@ static int plan_rows(const mla_attn_args * a, Plan * pl, int64_t all_rows, bool 
     // split the KV range so that about two workgroups per CU exist (256 CUs), in units of whole pages
     int64_t n_pages = (max_len + MLA_PAGE_TOKENS - 1) / MLA_PAGE_TOKENS;
     if (n_pages < 1) n_pages = 1;
-    int64_t splits = a->n_splits;
+    int64_t splits = a->n_splits, f32_max = PART_F32_MAX;
     if (splits == 0) {
         const int64_t wgs = (int64_t) a->n_seq * pl->n_row_blocks;
         splits = (256 + wgs - 1) / wgs;
         if (pl->wd > 1) splits *= 2;  // small-row shapes leave room for two workgroups per CU
+        const int64_t n_tiles = (max_len + TILE_TOK - 1) / TILE_TOK;
+        if (frugal == 2 && pl->variant == 2 && a->mask && n_rows > 32 && wgs < 256 && (a->n_seq > 1 || a->block_table)) splits = masked_splits(wgs, n_tiles, 32);
         if (pl->variant == 2 && a->mask && !frugal) {
-            const int64_t n_tiles = (max_len + TILE_TOK - 1) / TILE_TOK;
             if (n_rows <= 32)   splits = std::max<int64_t>(256 / wgs, 1);   // (the k-split program: short pieces, and no second round for the rest)
             else if (a->n_seq == 1 && !a->block_table) { if (!masked_worth_dealing(wgs, n_tiles)) splits = 1; }
             else if (wgs < 256) {
-                // (partials that are f32 with a workgroup for every CU stay f32: no more splits than that allows)
-                const int64_t split_bytes = (int64_t) a->n_seq * n_rows * 512 * sizeof(float), fill_pages = (n_pages + splits - 1) / splits;
-                const bool f32 = (n_pages + fill_pages - 1) / fill_pages * split_bytes <= PART_F32_MAX;
-                splits = masked_splits(wgs, n_tiles, f32 ? std::min<int64_t>(32, PART_F32_MAX / split_bytes) : 32);
+                // As many splits as pay: up to 32, or a workgroup for every CU where that takes more (a step of few tokens behind a long context).
+                // What is f32 with 32 splits, or with a workgroup for every CU, is f32 with more of them too: 4 row blocks x 32768 keys in
+                // 32 / 64 pieces 71 / 68 us (64 of f16: 59), 1 x 32768 in 32 / 128 / 256 63 / 41 / 48 (256 of f16: 44).
+                const int64_t split_bytes = (int64_t) a->n_seq * n_rows * 512 * sizeof(float), fill = splits;
+                auto in_pages = [&](int64_t s) { const int64_t per = (n_pages + s - 1) / s; return (n_pages + per - 1) / per; };
+                splits = masked_splits(wgs, n_tiles, 32);
+                const bool f32 = std::min(in_pages(splits), in_pages(fill)) * split_bytes <= PART_F32_MAX;
+                if (f32) f32_max = 2 * PART_F32_MAX;
+                const int64_t most = f32 ? std::min(fill, f32_max / split_bytes) : fill;
+                if (f32 && splits * split_bytes > f32_max) splits = std::max<int64_t>(f32_max / split_bytes, 1);
+                if (most > 32) {   // (from 8 % on: 1 row block x 8192 keys in 32 / 64 pieces 34 / 36.5 us, 2 of 48 rows 34.7 / 31)
+                    const double  merge = f32 ? 0.08 * std::min<int64_t>(n_rows, 128) / 128 : 0.01;
+                    const int64_t more  = masked_splits(wgs, n_tiles, most, merge, splits);
+                    if (masked_split_cost(wgs, n_tiles, more, merge) < 0.92 * masked_split_cost(wgs, n_tiles, splits, merge)) splits = more;
+                }
             }
             // More row blocks than whole rounds of 256 take: the ones left over would have the chip to themselves with most of it idle
             // (333 row blocks x 130 tiles: the 77 of the second round took nearly as long as the 256 of the first).  They are split, the
@@ -1178,7 +1190,7 @@ static int plan_rows(const mla_attn_args * a, Plan * pl, int64_t all_rows, bool 
         const size_t slot_rows = pl->balanced == 2 || pl->tail_splits ? 128 : (size_t) n_rows;
         const size_t n_part = n_slots * slot_rows * (pl->variant == 2 ? 512 : a->dv);
         // (a tail's rows would be whole without it, with no partial at all: theirs are f32 at any size)
-        pl->part_f32   = pl->tail_splits || n_part * sizeof(float) <= (size_t) PART_F32_MAX;
+        pl->part_f32   = pl->tail_splits || (int64_t) (n_part * sizeof(float)) <= f32_max;
         pl->ws_part_o  = n_part * (pl->part_f32 ? sizeof(float) : sizeof(_Float16));
         pl->ws_part_ml = n_slots * slot_rows * 2 * sizeof(float);
     }
@@ -1241,7 +1253,7 @@ int mla_attn_plan(const mla_attn_args * args, mla_attn_plan_info * out) {
 
 // phases: bit 0 = the attention kernels (partials or final output), bit 1 = the combine pass,
 // bit 2 = the small passes ahead of the pipelined kernel (Q operand image, key extent of the mask)
-static int launch_phases(const mla_attn_args * args, void * stream, int phases, bool frugal = false) {
+static int launch_phases(const mla_attn_args * args, void * stream, int phases, int frugal = 0) {
     Plan pl;
     const int rc = make_plan(args, &pl, frugal);
     if (rc) return rc;
@@ -1417,9 +1429,8 @@ int mla_attn_launch_static(const mla_attn_args * a, void * stream) {
     b.workspace      = nullptr;
     b.workspace_size = 0;
     Plan pl;
-    int rc = make_plan(&b, &pl);
-    const bool frugal = !rc && plan_ws(pl) > MLA_ATTN_STATIC_WORKSPACE_MAX;
-    if (frugal) rc = make_plan(&b, &pl, true);
+    int rc = make_plan(&b, &pl), frugal = 0;
+    while (!rc && plan_ws(pl) > MLA_ATTN_STATIC_WORKSPACE_MAX && frugal < 2) rc = make_plan(&b, &pl, ++frugal);
     if (rc) return rc;
     if (plan_ws(pl) > MLA_ATTN_STATIC_WORKSPACE_MAX) return MLA_ERR_TOO_LARGE;
     b.workspace      = ptr;

@@ -86,3 +86,9 @@ def test_more_splits_of_a_masked_launch_keep_f32_partials(n_seq, n_tok, n_head, 
     kw = dict(paged=paged, mask_width=keys)
     splits, rows = _plan(n_seq, n_tok, n_head, keys, F16, **kw).n_splits, n_tok * n_head
     assert splits > 1 and _workspace(n_seq, n_tok, n_head, keys, F16, **kw) >= n_seq * splits * rows * 512 * 4
+@pytest.mark.parametrize("n_seq,n_tok,n_head,kv_type", [(1, 2, 64, BF16), (2, 8, 16, BF16), (1, 8, 16, Q8_0), (1, 4, 128, F16), (7, 1, 128, BF16)])
+def test_few_tokens_behind_a_long_context_fill_the_chip(n_seq, n_tok, n_head, kv_type):
+    """Masked row blocks over pages: 32 workgroups each leave most CUs idle."""
+    blocks = n_seq * ((n_tok * n_head + 127) // 128)
+    assert 128 <= _plan(n_seq, n_tok, n_head, 65536, kv_type, mask_width=65536).n_workgroups <= 256 + blocks
+    assert _plan(n_seq, n_tok, n_head, 2048, kv_type, mask_width=2048).n_workgroups == 16 * blocks   # a page each
