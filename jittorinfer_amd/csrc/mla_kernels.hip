@@ -1145,7 +1145,9 @@ static int plan_rows(const mla_attn_args * a, Plan * pl, int64_t all_rows, int f
         // the general kernel visits only the key range the mask leaves open, when the extent pass can read the mask rows
         // (8-byte loads over whole groups of 8 keys)
         const int64_t nk = key_capacity(a);
-        if (nk % 8 == 0 && !(a->mask_nb1 & 7) && !((uintptr_t) a->mask & 7))
+        // (a frugal plan has no extents of masks narrower than the cache, whose launches never had: 128 bytes per 128 rows)
+        const bool narrow = a->mask_ne0 < (a->block_table ? a->bt_stride * MLA_PAGE_TOKENS : a->n_kv);
+        if (nk % 8 == 0 && !(a->mask_nb1 & 7) && !((uintptr_t) a->mask & 7) && !(frugal && narrow))
             pl->ws_maskext = (size_t) ((n_rows + 127) / 128) * 16 * 2 * sizeof(int);
     }
     // A paged decode batch (one row block per sequence, no mask) that needs KV splits anyway: the pipelined kernel's

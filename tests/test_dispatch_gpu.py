@@ -232,3 +232,28 @@ def test_more_masked_sequences_than_workgroups(gpu, k_type, n_seq, n_head, n_new
     got = _run(gpu, q, k, k_type, mask=mask, scale=U.SCALE, **kw)[..., :512]
     for b in (0, 255, 256, n_seq - 1):
         print(b, U.check(got[b:b + 1], _want(q[b:b + 1], [cells(b)], k_type, mask), "sequence %d" % b))
+
+
+@pytest.mark.parametrize("k_type,n_seq,n_new,n_head,n_pages,width", [
+    (O.TYPE_Q8_0, 1, 381, 64, 75, 9504),      # 48 MB less 3 KB of partial rows on the general kernel: no room for mask extents
+    (O.TYPE_F16, 157, 3, 16, 93, 93 * 128),   # three splits in f16 fit, the two that fill the chip in f32 do not
+])
+def test_static_scratch_takes_what_only_the_smallest_plan_fits(gpu, k_type, n_seq, n_new, n_head, n_pages, width):
+    import ctypes as C
+    import torch
+    import jittorinfer_amd as J
+    rng = np.random.default_rng(n_new)
+    q = torch.from_numpy(rng.standard_normal((n_seq, n_head, n_new, 576)).astype(np.float32)).to(gpu)
+    pool = U.encode_kv(rng.standard_normal((n_pages * 128, 576)).astype(np.float32), k_type, q8_scale=1.0 / 32 if k_type == O.TYPE_Q8_0 else None)
+    k = torch.from_numpy(pool.view(np.int16) if pool.dtype == np.uint16 else pool).to(gpu)
+    bt = np.stack([rng.permutation(n_pages) for _ in range(n_seq)]).astype(np.int32)   # (one pool of pages that all the sequences share)
+    kw = dict(block_table=torch.from_numpy(bt).to(gpu), seq_lens=torch.full((n_seq,), width - 3, dtype=torch.int32, device=gpu))
+    mask = torch.from_numpy(_causal_mask(n_new, width - 3, width).view(np.float16)).to(gpu)
+    out = torch.full((n_seq, n_new, n_head, 512), float("nan"), dtype=torch.float32, device=gpu)
+    a, _, keep = J.capi.make_args(q, k, k_type, dv=512, scale=U.SCALE, mask=mask, out=out, **kw)
+    assert a.workspace_size > J.capi.MLA_ATTN_STATIC_WORKSPACE_MAX
+    a.workspace, a.workspace_size = None, 0
+    assert J.library().mla_attn_launch_static(C.byref(a), C.c_void_p(torch.cuda.current_stream(gpu).cuda_stream)) == 0
+    want = J.ggml_flash_attn_ext(q, k, k_type, dv=512, scale=U.SCALE, mask=mask, **kw)
+    torch.cuda.synchronize()
+    print(U.check(out.cpu().numpy(), want.cpu().numpy()[..., :512], "fixed scratch"))
