@@ -1177,13 +1177,21 @@ static hipError_t launch_variant(const KParams & kp, dim3 grid, hipStream_t st) 
 constexpr int64_t STREAM_CACHE_BYTES = 96ll << 20;   // (three times what the eight L2s hold)
 
 // Launches whose blocks of 128 rows are full, or of which at most the last one is not: its waves without rows compute on copies of the
-// last row (or on what the image holds) and nothing of theirs is stored.  The row-split program leaves such waves idle, but it is the slower one on every full
-// block, and it takes an operand image (2 sequences x 537 tokens x 64 heads, 64 rows over: 172 -> 117 us).  A single block of 65 to
-// 96 rows runs as fast on either (32 sequences x 8192 keys: 80 heads 101.6 / 100.7 us, 96 heads 102.3 / 103.4): it stays there.
+// last row (or on what the image holds) and nothing of theirs is stored.  The row-split program leaves such waves idle, but it is the
+// slower one on every full block of bf16 cells, which it converts, and it always takes an operand image.  Last block not full, row-split /
+// column-split, us: bf16 96 sequences x 224 rows x 4096 keys 297 / 255, 1 x 300 tokens x 24 heads x 16384 294 / 253, 10 x 160 x 13472 93 / 84.
+// f16 cells: unsplit masked launches (96 x 224 x 4096 239 / 227, 96 x 528 x 512 127 / 103) and long runs dealt out (1 x 300 tokens x 24
+// heads x 16384 261 / 253, but 1 x 2080 rows x 1024 40.5 / 42), not uniform splits (10 x 160 x 13472 77 / 88, 4 x 192 x 768 26.8 / 27.8);
+// without a mask only where few keys leave the operands to weigh most or the last block is a small part (96 x 288 x 512 90 / 80,
+// 96 x 528 x 4096 504 / 480; 96 x 160 x 4096 225 / 239).
+// A single block of 65 to 96 rows runs as fast on either (32 sequences x 8192 keys: 80 heads 101.6 / 100.7, 96 heads 102.3 / 103.4): it
+// stays on the row-split one.
 static bool decode_cs_applicable(const KParams & kp, int kv_type) {
     if (kv_type != MLA_TYPE_BF16 && kv_type != MLA_TYPE_F16) return false;
-    if (kp.bf16_direct || kp.q_as_q8) return false;
-    return decode_cs_rows(kp.n_rows) && kp.slot_rows < (1 << 22);
+    if (kp.bf16_direct || kp.q_as_q8 || !decode_cs_rows(kp.n_rows) || kp.slot_rows >= (1 << 22)) return false;
+    const int tail = kp.n_rows % 128;
+    if (kv_type == MLA_TYPE_BF16 || tail == 0 || tail > 96) return true;
+    return kp.n_splits == 1 ? kp.mask || kp.key_cap <= 1024 || kp.n_rows > 512 : kp.balanced == 2 && kp.split_tokens >= 512;   // (a tail: masked, unsplit)
 }
 
 // 33 .. 64 rows per sequence (a decode step of a model with 48 or 64 heads per device), no mask: the column-split program for two row

@@ -257,3 +257,22 @@ def test_static_scratch_takes_what_only_the_smallest_plan_fits(gpu, k_type, n_se
     want = J.ggml_flash_attn_ext(q, k, k_type, dv=512, scale=U.SCALE, mask=mask, **kw)
     torch.cuda.synchronize()
     print(U.check(out.cpu().numpy(), want.cpu().numpy()[..., :512], "fixed scratch"))
+
+
+@pytest.mark.parametrize("k_type", [O.TYPE_BF16, O.TYPE_F16])
+@pytest.mark.parametrize("n_seq,n_head,n_new,n_kv", [(96, 16, 33, 288), (96, 16, 33, 1056), (128, 48, 3, 288), (128, 48, 3, 1056)])   # 528 and 144 rows
+@pytest.mark.parametrize("masked", [False, True])
+def test_unsplit_row_blocks_of_which_the_last_is_not_full(gpu, k_type, n_seq, n_head, n_new, n_kv, masked):
+    """A workgroup per row block; f16 cells stay on the row-split program without a mask, over more than 1024 cells and up to 512 rows.  (The
+    sequences share one cache: their stride is 0.)"""
+    import torch
+    import jittorinfer_amd as J
+    rng = np.random.default_rng(n_head * n_kv)
+    q = rng.standard_normal((n_seq, n_head, n_new, 576)).astype(np.float32)
+    k = U.encode_kv(rng.standard_normal((1, n_kv, 576)).astype(np.float32), k_type)
+    mask = _causal_mask(n_new, n_kv, n_kv) if masked else None
+    kw = dict(mask=torch.from_numpy(mask.view(np.float16)).to(gpu)) if masked else {}
+    assert J.plan(torch.from_numpy(q).to(gpu), torch.from_numpy(k.view(np.int16)).to(gpu), k_type, scale=U.SCALE, **kw)["n_splits"] == 1
+    got = _run(gpu, q, k, k_type, mask=mask, scale=U.SCALE)[..., :512]
+    for b in (0, n_seq - 1):
+        print(b, U.check(got[b:b + 1], _want(q[b:b + 1], [k[0]], k_type, mask), "sequence %d" % b))
