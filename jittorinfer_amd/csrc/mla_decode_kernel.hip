@@ -309,14 +309,16 @@ __device__ __forceinline__ void decode_body() {
     int bx = blockIdx.x, by = blockIdx.y, bz = blockIdx.z;
     bool tail = false;   // this workgroup has one of several pieces of a row block of the launch's tail
     if constexpr (TAIL) {
-        // Row blocks in their natural order, short ones of a causal chunk first: the XCDs get the same share of every sequence (runs of
-        // neighbours per XCD do not, where there are several sequences), and workgroups that run together read the same keys at about the
-        // same time, which the folded order below does not keep up over several rounds.  Runs of neighbours folded for one sequence /
-        // natural, us: 3 x 1467 tokens x 32 heads Q8_0 513 / 446, 2 x 1974 x 128 2307 / 1840, 1 x 1603 x 64 681 / 640, 1 x 333 x 128 behind
-        // 4000 383 / 378, 16 x 657 x 16 430 / 431.
+        // Row blocks in their natural order, short ones of a causal chunk first: the XCDs get the same share of every sequence, and
+        // workgroups that run together read the same keys at about the same time, which the folded order below does not keep up over
+        // several rounds.  Runs of neighbours per XCD, folded for one sequence / natural, us: 3 x 1467 tokens x 32 heads Q8_0 513 / 446,
+        // 2 x 1974 x 128 2307 / 1840, 1 x 1603 x 64 681 / 640, 1 x 333 x 128 behind 4000 383 / 378, 16 x 657 x 16 430 / 431.
+        // Sequences of few row blocks, of which such a run holds four or more whole ones, keep the runs: their blocks share an XCD's L2
+        // (44 sequences x 8 row blocks x 7584 keys 721 / 744, 40 x 8 x 4096 379 / 394, 96 x 3 x 4096 366 / 374).
         const int n_rb = (p.n_rows + 127) / 128, id = blockIdx.x;
         tail = id >= p.tail_first;
-        const int item = tail ? p.tail_first + (id - p.tail_first) / p.tail_splits : id;
+        const int item = tail ? p.tail_first + (id - p.tail_first) / p.tail_splits
+                       : 32 * n_rb <= p.tail_first ? (id & 7) * (p.tail_first >> 3) + (id >> 3) : id;
         bx = tail ? (id - p.tail_first) % p.tail_splits : 0;
         bz = item / n_rb; by = item - bz * n_rb;
     } else {
