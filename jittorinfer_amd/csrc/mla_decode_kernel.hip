@@ -1184,6 +1184,7 @@ constexpr int64_t STREAM_CACHE_BYTES = 96ll << 20;   // (three times what the ei
 // column-split, us: bf16 96 sequences x 224 rows x 4096 keys 297 / 255, 1 x 300 tokens x 24 heads x 16384 294 / 253, 10 x 160 x 13472 93 / 84.
 // f16 cells: unsplit masked launches (96 x 224 x 4096 239 / 227, 96 x 528 x 512 127 / 103) and long runs dealt out (1 x 300 tokens x 24
 // heads x 16384 261 / 253, but 1 x 2080 rows x 1024 40.5 / 42), not uniform splits (10 x 160 x 13472 77 / 88, 4 x 192 x 768 26.8 / 27.8);
+// a page of keys only from 64 row blocks on (8 x 160 x 128 25.5 / 27.3, 32 x 144 x 128 30.7 / 28.1),
 // without a mask only where few keys leave the operands to weigh most or the last block is a small part (96 x 288 x 512 90 / 80,
 // 96 x 528 x 4096 504 / 480; 96 x 160 x 4096 225 / 239).
 // A single block of 65 to 96 rows runs as fast on either (32 sequences x 8192 keys: 80 heads 101.6 / 100.7, 96 heads 102.3 / 103.4): it
@@ -1193,7 +1194,9 @@ static bool decode_cs_applicable(const KParams & kp, int kv_type) {
     if (kp.bf16_direct || kp.q_as_q8 || !decode_cs_rows(kp.n_rows) || kp.slot_rows >= (1 << 22)) return false;
     const int tail = kp.n_rows % 128;
     if (kv_type == MLA_TYPE_BF16 || tail == 0 || tail > 96) return true;
-    return kp.n_splits == 1 ? kp.mask || kp.key_cap <= 1024 || kp.n_rows > 512 : kp.balanced == 2 && kp.split_tokens >= 512;   // (a tail: masked, unsplit)
+    if (kp.n_splits > 1) return kp.balanced == 2 && kp.split_tokens >= 512;
+    if (!kp.mask) return kp.key_cap <= 1024 || kp.n_rows > 512;
+    return kp.key_cap > 128 || kp.n_seq_sched * ((kp.n_rows + 127) / 128) >= 64;   // (any launch with a tail)
 }
 
 // 33 .. 64 rows per sequence (a decode step of a model with 48 or 64 heads per device), no mask: the column-split program for two row

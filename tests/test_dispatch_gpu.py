@@ -276,3 +276,13 @@ def test_unsplit_row_blocks_of_which_the_last_is_not_full(gpu, k_type, n_seq, n_
     got = _run(gpu, q, k, k_type, mask=mask, scale=U.SCALE)[..., :512]
     for b in (0, n_seq - 1):
         print(b, U.check(got[b:b + 1], _want(q[b:b + 1], [k[0]], k_type, mask), "sequence %d" % b))
+
+
+@pytest.mark.parametrize("n_seq,n_head,n_new", [(8, 16, 10), (31, 16, 10), (32, 16, 10)])   # 16, 62 and 64 row blocks
+def test_one_page_of_f16_keys_behind_a_mask(gpu, n_seq, n_head, n_new):
+    """Two row blocks per sequence, the second of 32 rows: the row-split program below 64 row blocks, the column-split one from there on."""
+    rng = np.random.default_rng(n_seq)
+    q = rng.standard_normal((n_seq, n_head, n_new, 576)).astype(np.float32)
+    k = U.encode_kv(rng.standard_normal((n_seq, 128, 576)).astype(np.float32), O.TYPE_F16)
+    mask = _causal_mask(n_new, 128, 128)
+    print(U.check(_run(gpu, q, k, O.TYPE_F16, mask=mask, scale=U.SCALE)[..., :512], _want(q, list(k), O.TYPE_F16, mask), "one page"))
