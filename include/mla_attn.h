@@ -62,7 +62,7 @@ extern "C" {
                                       0 or in [2^-14, 65504] (bf16 has fewer mantissa bits than f16), larger ones become
                                       +-65504, smaller ones lose bits below 2^-24; probabilities are rounded to f16.  Set it
                                       for a cache that holds values outside that range.  Without it, too, the tiles are multiplied
-                                      as they are where mask rows end before the block table's last page does. */
+                                      as they are where mask rows end before the cache or the block table's last page does. */
 
 /* errors */
 #define MLA_ERR_BAD_SHAPE     (-1)
@@ -71,7 +71,7 @@ extern "C" {
 #define MLA_ERR_WORKSPACE     (-4)
 #define MLA_ERR_NULL          (-5)
 #define MLA_ERR_UNSUPPORTED   (-6)
-#define MLA_ERR_TOO_LARGE     (-7) /* mla_attn_launch_static: the call needs more scratch than MLA_ATTN_STATIC_WORKSPACE_MAX */
+#define MLA_ERR_TOO_LARGE     (-7) /* mla_attn_launch_static: the call cannot do with MLA_ATTN_STATIC_WORKSPACE_MAX bytes of scratch */
 
 #define MLA_PAGE_TOKENS 128
 
@@ -166,9 +166,9 @@ int    mla_attn_launch_kernel(const mla_attn_args * args, void * stream);
 /* mla_attn_launch with the library's own scratch instead of `workspace` (args->workspace and workspace_size are ignored).
  * No counterpart in the reference.  For callers that cannot allocate device memory around the call: code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc.  The scratch is a fixed array of
- * MLA_ATTN_STATIC_WORKSPACE_MAX bytes that every device the library runs on holds until the process ends; a call whose
- * mla_attn_workspace_size() exceeds it returns MLA_ERR_TOO_LARGE (the headline decode step, 32 sequences x 128 heads x 8192
- * keys, needs 43 MB).  Allocates nothing.  All calls on one device share the array: calls that overlap in time on the same
+ * MLA_ATTN_STATIC_WORKSPACE_MAX bytes that every device the library runs on holds until the process ends.  A call whose
+ * mla_attn_workspace_size() exceeds it (the headline decode step, 32 sequences x 128 heads x 8192 keys, needs 43 MB) runs without the
+ * scratch that only saves time, and returns MLA_ERR_TOO_LARGE where the rest does not fit either.  Allocates nothing.  All calls on one device share the array: calls that overlap in time on the same
  * device (different streams or threads) race; calls on one stream, or otherwise ordered, do not. */
 #define MLA_ATTN_STATIC_WORKSPACE_MAX ((size_t) 48 << 20)
 int    mla_attn_launch_static(const mla_attn_args * args, void * stream);

@@ -907,7 +907,7 @@ struct Plan {
     int    balanced, n_wg, n_units;   // balanced schedule of the pipelined kernel (1: ragged paged decode, 2: masked launch)
     int    dual;                      // the masked launch is issued in two forms, see token_form_candidate
     int    tail_first, tail_splits;   // masked launch beyond whole rounds of workgroups: see masked_splits
-    int    seq_shift;                 // heads in 2^seq_shift groups, each a "sequence" of the launch: see head_groups
+    int    seq_shift;                 // heads in 2^seq_shift groups, each a "sequence" of the launch: see head_groups_shift
     int    seq_sorted;                // paged decode of more than 256 sequences: workgroups take the sequences longest first
 };
 
@@ -985,6 +985,7 @@ static int64_t masked_splits(int64_t n_items, int64_t n_tiles, int64_t most, dou
 // One sequence in a contiguous cache, whose split form is the schedule that deals out equal runs of tiles: worth it from this many on.
 // 16 heads, a workgroup per row block / runs dealt out: 8 row blocks x 18 tiles 45.0 / 42.8 us, 32 x 8 33.3 / 43.8, 64 x 16 43.1 / 47.2, 64 x 32
 // 64.8 / 49.9, 128 x 64 110 / 99, 160 x 40 79 / 163, 160 x 168 252 / 236, 192 x 112 187 / 193, 250 x 63 119 / 281, 250 x 319 581 / 624.
+// Q8_0 cells would gain from fewer tiles on (55 x 14 tiles 51.0 / 46.0, 77 x 14 52.7 / 50.9), but whole rows are never rounded to 16 bits in between.
 static bool masked_worth_dealing(int64_t n_items, int64_t n_tiles) {
     return n_items <= 8 ? n_tiles > 4 : n_tiles * (1280 - 6 * n_items) > 15360;   // (2 x 10 35.1 / 25.2, 4 x 5 28.1 / 24.9, 8 x 6 29.6 / 28.2, 16 x 8 33.3 / 33.9)
 }
