@@ -389,9 +389,12 @@ PyObject * bind(PyObject *, PyObject * const * v, Py_ssize_t n) {
 }
 
 template <PyObject * (*F)(PyObject *, PyObject * const *, Py_ssize_t)> PyObject * entry(PyObject * self, PyObject * const * v, Py_ssize_t n) {
-    HANDLE_TH_ERRORS
-    return F(self, v, n);
-    END_HANDLE_TH_ERRORS
+    try {
+        return F(self, v, n);
+    } catch (...) {   // (what HANDLE_TH_ERRORS does, without its buffer for torch's warnings: none arise here)
+        torch::translate_exception_to_python(std::current_exception());
+        return nullptr;
+    }
 }
 
 #define FAST(name) { #name, (PyCFunction) (void (*)(void)) entry<name>, METH_FASTCALL, nullptr }

@@ -34,6 +34,7 @@ calls = dict(
     kv_write_rope=lambda: J.kv_write(rows, cache, J.MLA_TYPE_BF16, row0=0, stream=0, k_pe=rows[:, 512:], rope=dict(pos=sparse, n_dims=64)),
     copy=lambda: J.copy_f32(x, torch.zeros((4, 16, 64)).to_sparse(), stream=0),
 )
+J.capi.native()   # (a module that does not load is no error of a call)
 seen = {}
 for name, call in calls.items():
     try:
