@@ -1018,7 +1018,8 @@ static mla_attn_args grouped(const mla_attn_args * a, int shift) {
 }
 
 // frugal: for a caller whose scratch is fixed -- no partial rows that only save time (no groups of heads, no tail, as many splits of a
-// masked launch as give every CU a workgroup, or with 2 as few of those as pay; narrow masks on the kernel that needs no operand image).
+// masked launch as give every CU a workgroup, or with 2 as few of those as pay; narrow masks on the kernel that needs no operand image,
+// with 3 and a contiguous cache in one split).
 int make_plan(const mla_attn_args * a, Plan * pl, int frugal = 0) {
     const int rc = validate(a);
     if (rc) return rc;
@@ -1078,6 +1079,7 @@ static int plan_rows(const mla_attn_args * a, Plan * pl, int64_t all_rows, int f
         splits = (256 + wgs - 1) / wgs;
         if (pl->wd > 1) splits *= 2;  // small-row shapes leave room for two workgroups per CU
         const int64_t n_tiles = (max_len + TILE_TOK - 1) / TILE_TOK;
+        if (frugal == 3 && a->mask && !a->block_table && a->mask_ne0 < a->n_kv) splits = 1;
         if (frugal == 2 && pl->variant == 2 && a->mask && n_rows > 32 && wgs < 256 && (a->n_seq > 1 || a->block_table)) splits = masked_splits(wgs, n_tiles, 32);
         if (pl->variant == 2 && a->mask && !frugal) {
             if (n_rows <= 32)   splits = std::max<int64_t>(256 / wgs, 1);   // (the k-split program: short pieces, and no second round for the rest)
@@ -1433,7 +1435,7 @@ int mla_attn_launch_static(const mla_attn_args * a, void * stream) {
     b.workspace_size = 0;
     Plan pl;
     int rc = make_plan(&b, &pl), frugal = 0;
-    while (!rc && plan_ws(pl) > MLA_ATTN_STATIC_WORKSPACE_MAX && frugal < 2) rc = make_plan(&b, &pl, ++frugal);
+    while (!rc && plan_ws(pl) > MLA_ATTN_STATIC_WORKSPACE_MAX && frugal < 3) rc = make_plan(&b, &pl, ++frugal);
     if (rc) return rc;
     if (plan_ws(pl) > MLA_ATTN_STATIC_WORKSPACE_MAX) return MLA_ERR_TOO_LARGE;
     b.workspace      = ptr;

@@ -286,3 +286,23 @@ def test_one_page_of_f16_keys_behind_a_mask(gpu, n_seq, n_head, n_new):
     k = U.encode_kv(rng.standard_normal((n_seq, 128, 576)).astype(np.float32), O.TYPE_F16)
     mask = _causal_mask(n_new, 128, 128)
     print(U.check(_run(gpu, q, k, O.TYPE_F16, mask=mask, scale=U.SCALE)[..., :512], _want(q, list(k), O.TYPE_F16, mask), "one page"))
+
+
+def test_static_scratch_takes_a_chunk_behind_a_mask_narrower_than_its_cache(gpu):
+    """25600 rows over a contiguous cache: the f16 partial rows of two splits do not fit the fixed scratch, whole rows need none."""
+    import ctypes as C
+    import torch
+    import jittorinfer_amd as J
+    rng = np.random.default_rng(17)
+    n_new, n_head, n_kv, width = 200, 128, 1024, 992
+    q = torch.from_numpy(rng.standard_normal((1, n_head, n_new, 576)).astype(np.float32)).to(gpu)
+    k = torch.from_numpy(U.encode_kv(rng.standard_normal((1, n_kv, 576)).astype(np.float32), O.TYPE_BF16).view(np.int16)).to(gpu)
+    mask = torch.from_numpy(_causal_mask(n_new, width - 5, width).view(np.float16)).to(gpu)
+    out = torch.full((1, n_new, n_head, 512), float("nan"), dtype=torch.float32, device=gpu)
+    a, _, keep = J.capi.make_args(q, k, O.TYPE_BF16, dv=512, scale=U.SCALE, mask=mask, out=out)
+    assert a.workspace_size > J.capi.MLA_ATTN_STATIC_WORKSPACE_MAX
+    a.workspace, a.workspace_size = None, 0
+    assert J.library().mla_attn_launch_static(C.byref(a), C.c_void_p(torch.cuda.current_stream(gpu).cuda_stream)) == 0
+    want = J.ggml_flash_attn_ext(q, k, O.TYPE_BF16, dv=512, scale=U.SCALE, mask=mask)
+    torch.cuda.synchronize()
+    print(U.check(out.cpu().numpy(), want.cpu().numpy()[..., :512], "fixed scratch"))
